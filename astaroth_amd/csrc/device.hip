@@ -148,6 +148,8 @@ static void make_phys(const AcMeshInfo& info, PhysParams<AcReal>& P)
     P.gamma_inv_cp = (AcReal)(gamma / cp);
     P.eta_mu0 = (AcReal)((double)info.real_params[AC_eta] * mu0);
     P.nu_third = (AcReal)((double)info.real_params[AC_nu_visc] / 3.0);
+    P.nu_third_zeta = (AcReal)((double)info.real_params[AC_nu_visc] / 3.0 +
+                               (double)info.real_params[AC_zeta]);
     P.pT_scale = (AcReal)(cs * cs * exp(-(double)info.real_params[AC_lnT0]));
 }
 
@@ -190,6 +192,9 @@ static void fill_solve_args(Device d, SolveArgs<AcReal>& a, int step, AcReal dt)
     a.fstride = (long long)d->count;
     a.C = d->C;
     make_phys(info, a.P);
+    for (int p = 0; p < 3; ++p)
+        for (int o = 0; o < 4; ++o)
+            a.mxv[p][o] = (AcReal)((double)a.P.nu_third_zeta * (double)a.C.mx[p][o]);
     const AcReal alpha[3] = {(AcReal)0.0, (AcReal)(-5.0 / 9.0), (AcReal)(-153.0 / 128.0)};
     const AcReal beta[3] = {(AcReal)(1.0 / 3.0), (AcReal)(15.0 / 16.0), (AcReal)(8.0 / 15.0)};
     a.dt = dt;
@@ -207,9 +212,12 @@ static void fill_solve_args(Device d, SolveArgs<AcReal>& a, int step, AcReal dt)
 }
 
 // Launch shapes: kind 0 runs the delay-line (or ring) kernel of solve_tiled.hip, kind 1 the
-// unrolled sweep of solve_sweep.hip; tx == 0 is the direct kernel.
+// unrolled sweep of solve_sweep.hip, kind 2 the role-split kernel of solve_split.hip; tx == 0 is
+// the direct kernel.
 static bool shape_fits(TiledShape s, int3 n)
 {
+    if (s.kind == 2)
+        return split_shape_fits(s, n.x, n.y, n.z);
     return s.kind == 1 ? sweep_shape_fits(s, n.x, n.y, n.z) : tiled_shape_fits(s, n.x, n.y, n.z);
 }
 
@@ -218,6 +226,8 @@ static bool shape_reads_periodic(const SolveArgs<AcReal>& a, int kb, TiledShape 
 {
     if (s.tx <= 0)
         return false;
+    if (s.kind == 2)
+        return split_reads_periodic<AcReal>(a, kb, s);
     return s.kind == 1 ? sweep_applies<AcReal>(a, kb, s) : tiled_reads_periodic<AcReal>(a, kb, s);
 }
 
@@ -226,6 +236,8 @@ static bool launch_shape(const SolveArgs<AcReal>& a, bool upwd, bool entropy, in
 {
     if (s.tx <= 0)
         return false;
+    if (s.kind == 2)
+        return launch_solve_split<AcReal>(a, upwd, entropy, kb, s, st);
     return s.kind == 1 ? launch_solve_sweep<AcReal>(a, upwd, entropy, kb, s, st)
                        : launch_solve_tiled<AcReal>(a, upwd, entropy, kb, s, st);
 }
@@ -234,7 +246,10 @@ static bool launch_shape(const SolveArgs<AcReal>& a, bool upwd, bool entropy, in
 static TiledShape config_shape(const AcMeshInfo& c)
 {
     return TiledShape{c.int_params[AC_solve_tile_x], c.int_params[AC_solve_tile_y],
-                      c.int_params[AC_solve_zchunk], c.int_params[AC_solve_kernel] == 1 ? 1 : 0};
+                      c.int_params[AC_solve_zchunk],
+                      c.int_params[AC_solve_kernel] == 1 || c.int_params[AC_solve_kernel] == 2
+                          ? c.int_params[AC_solve_kernel]
+                          : 0};
 }
 
 static AcResult launch_solve(Device d, const SolveArgs<AcReal>& a_in, hipStream_t s)
@@ -465,7 +480,8 @@ AcResult acDevicePrintInfo(const Device d)
            p.multiProcessorCount, p.totalGlobalMem / 1073741824.0);
     printf("  grid %d x %d x %d, AcReal %zu bytes, kahan bits %d, solve shape %d x %d x %d (%s)\n",
            n.x, n.y, n.z, sizeof(AcReal), d->kahan_bits, d->shape.tx, d->shape.ty, d->shape.zchunk,
-           d->shape.tx <= 0 ? "direct" : (d->shape.kind == 1 ? "sweep" : "delay-line"));
+           d->shape.tx <= 0 ? "direct"
+                            : (d->shape.kind == 2 ? "split" : (d->shape.kind == 1 ? "sweep" : "delay-line")));
     return AC_SUCCESS;
 }
 
@@ -1233,8 +1249,8 @@ AcResult acDeviceGetSolveKernel(const Device d, int* kind)
 }  // extern "C"
 
 // ------------------------------------------------------------------ autotuner
-// Times every candidate launch (the direct kernel, the delay-line shapes and the sweep shapes) on
-// the current grid with the device's own compensation width, physics switches and periodic-image
+// Times the candidate launches (listed in autotune below; a single one is taken untimed) on the
+// current grid with the device's own compensation width, physics switches and periodic-image
 // reads, and keeps the fastest. No allocation: the trial launches read the real state and write
 // f' into the out slab, which holds nothing between substeps. When the tuning runs ahead of a
 // substep-0 launch (every caller's first substep), w is dead as well -- that launch overwrites it
@@ -1247,6 +1263,13 @@ AcResult acDeviceGetSolveKernel(const Device d, int* kind)
 // cached in the file named by ASTAROTH_AUTOTUNE_CACHE (lines "nx ny nz kahan upwd entropy
 // realsize tx ty zchunk kind"); ASTAROTH_AUTOTUNE_VERBOSE=1 prints each candidate's time to
 // stderr.
+// AC_solve_kernel < 0 leaves the role-split kernel out of the trials; such choices are cached with a
+// twelfth value of 1, which other devices pass over.
+static bool column_kernels_only(Device d)
+{
+    return d->local_config.int_params[AC_solve_kernel] < 0;
+}
+
 static bool read_cache(Device d, TiledShape* out)
 {
     const char* path = getenv("ASTAROTH_AUTOTUNE_CACHE");
@@ -1259,9 +1282,11 @@ static bool read_cache(Device d, TiledShape* out)
     char line[256];
     bool found = false;
     while (fgets(line, sizeof(line), fp)) {
-        int v[11];
-        if (sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4],
-                   &v[5], &v[6], &v[7], &v[8], &v[9], &v[10]) != 11)
+        int v[12] = {};
+        if (sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4],
+                   &v[5], &v[6], &v[7], &v[8], &v[9], &v[10], &v[11]) < 11)
+            continue;
+        if (column_kernels_only(d) ? v[10] == 2 : v[11] != 0)
             continue;
         if (v[0] == n.x && v[1] == n.y && v[2] == n.z && v[3] == d->kahan_bits &&
             v[4] == d->local_config.bool_params[AC_lupwd] &&
@@ -1286,9 +1311,9 @@ static void write_cache(Device d, TiledShape s)
     if (!fp)
         return;
     const int3 n = d->local_config.int3_params[AC_nlocal];
-    fprintf(fp, "%d %d %d %d %d %d %d %d %d %d %d\n", n.x, n.y, n.z, d->kahan_bits,
+    fprintf(fp, "%d %d %d %d %d %d %d %d %d %d %d%s\n", n.x, n.y, n.z, d->kahan_bits,
             d->local_config.bool_params[AC_lupwd], d->local_config.bool_params[AC_lentropy],
-            (int)sizeof(AcReal), s.tx, s.ty, s.zchunk, s.kind);
+            (int)sizeof(AcReal), s.tx, s.ty, s.zchunk, s.kind, column_kernels_only(d) ? " 1" : "");
     fclose(fp);
 }
 
@@ -1328,7 +1353,37 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
         }
         ta[t].wrap = 1;
     }
-    const SolveArgs<AcReal>& a = ta[0];
+    // Candidates: the role-split shapes (any grid); in FP32 also the delay-line shapes of 64 x 4 columns
+    // that give each CU its two workgroups, which are faster once the state is far larger than the caches
+    // (256^3 plain: 0.54 against 0.59 ms per launch; smaller grids 0.105 against 0.079 ms at 128^3, and
+    // FP64 1.59 against 1.36 ms at 256^3); and the direct kernel up to 32^3 cells, where it is about as
+    // fast as the others (32^3 FP32: 0.0092 ms each). Where the configuration leaves the role-split
+    // kernel out: the direct kernel, the delay-line and the sweep shapes of 64 columns. The ring shapes
+    // read halos as stored and never win; they stay pinnable.
+    std::vector<TiledShape> cands;
+    TiledShape split[4];
+    const int nsplit = one_slab && !column_kernels_only(d) ? split_candidates(n.x, n.y, n.z, split, 4) : 0;
+    cands.assign(split, split + nsplit);
+    for (int i = 0; one_slab && i < tiled_num_shapes(); ++i) {
+        const TiledShape sh = tiled_shape(i);
+        if (sh.tx != 64 || !shape_fits(sh, n))
+            continue;
+        const long long blocks = (long long)(n.x / 64) * (n.y / sh.ty) * (n.z / sh.zchunk);
+        if (nsplit == 0 || (sizeof(AcReal) == 4 && sh.ty == 4 && blocks >= 512))
+            cands.push_back(sh);
+    }
+    if (one_slab && nsplit == 0)
+        for (const TiledShape& sh : kSweepShapes)
+            if (shape_fits(sh, n) && sweep_applies<AcReal>(ta[0], kb, sh))
+                cands.push_back(sh);
+    if (nsplit == 0 || (long long)n.x * n.y * n.z <= 32768)
+        cands.push_back(TiledShape{0, 0, 0, 0});
+    if (cands.size() == 1) {
+        d->shape = cands[0];
+        d->shape_tuned = true;
+        write_cache(d, d->shape);
+        return AC_SUCCESS;
+    }
     hipEvent_t e0, e1;
     AC_HIP_CHECK(hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -1345,8 +1400,11 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
                     ad.wrap = 0;  // the direct kernel reads the halos as stored
                     launch_solve_direct<AcReal>(ad, upwd, entropy, kb, s);
                 }
-                else if (!launch_shape(ta[t], upwd, entropy, kb, sh, s)) {
-                    return false;
+                else {
+                    SolveArgs<AcReal> at = ta[t];
+                    at.wrap = shape_reads_periodic(at, kb, sh) ? 1 : 0;
+                    if (!launch_shape(at, upwd, entropy, kb, sh, s))
+                        return false;
                 }
             }
             return true;
@@ -1372,19 +1430,6 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
                     best_ms / (2 * ntrial));
         return best_ms;
     };
-    std::vector<TiledShape> cands;
-    cands.push_back(TiledShape{0, 0, 0, 0});
-    if (one_slab) {
-        for (int i = 0; i < tiled_num_shapes(); ++i) {
-            const TiledShape sh = tiled_shape(i);
-            // the ring kernels read halos as stored and never win; they stay pinnable only
-            if (sh.tx == 64 && shape_fits(sh, n))
-                cands.push_back(sh);
-        }
-        for (const TiledShape& sh : kSweepShapes)
-            if (shape_fits(sh, n) && sweep_applies<AcReal>(a, kb, sh))
-                cands.push_back(sh);
-    }
     float best_ms = 1e30f;
     for (const TiledShape& sh : cands) {
         const float ms = time_candidate(sh);

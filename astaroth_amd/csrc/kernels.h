@@ -39,7 +39,9 @@ void launch_solve_direct(const SolveArgs<T>& a, bool upwd, bool entropy, int kah
 // 16 x 16 and 32 x 16 the four-plane ring kernel (solve_ring.hip).
 struct TiledShape {
     int tx, ty, zchunk;
-    int kind;  // 0: delay-line / ring kernel (solve_tiled.hip, solve_ring.hip); 1: sweep (solve_sweep.hip)
+    // 0: delay-line / ring kernel (solve_tiled.hip, solve_ring.hip); 1: sweep (solve_sweep.hip);
+    // 2: role-split (solve_split.hip)
+    int kind;
 };
 template <typename T>
 bool launch_solve_tiled(const SolveArgs<T>& a, bool upwd, bool entropy, int kahan_bits,
@@ -56,6 +58,15 @@ bool sweep_shape_fits(TiledShape s, int nx, int ny, int nz);
 // Whether launch_solve_sweep runs the sweep kernel for these arguments (it honours a.wrap).
 template <typename T>
 bool sweep_applies(const SolveArgs<T>& a, int kahan_bits, TiledShape shape);
+// The role-split kernel (solve_split.hip): any grid and z-chunk. Returns false (nothing launched) when
+// it does not apply.
+template <typename T>
+bool launch_solve_split(const SolveArgs<T>& a, bool upwd, bool entropy, int kahan_bits,
+                        TiledShape shape, hipStream_t stream);
+bool split_shape_fits(TiledShape s, int nx, int ny, int nz);
+int split_candidates(int nx, int ny, int nz, TiledShape* out, int max_out);
+template <typename T>
+bool split_reads_periodic(const SolveArgs<T>& a, int kahan_bits, TiledShape shape);
 // The adjoint's local stage on the tiled machinery: derivative adjoints g (NG fields of m^3,
 // same field stride as the state), lambda_f / lambda_w (NF fields, updated in place at the
 // interior cells: lambda_w <- alpha mu, lambda_f <- lambda_f + dt * the value adjoints), (nu, eta)

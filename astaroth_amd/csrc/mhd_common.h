@@ -22,6 +22,7 @@ struct PhysParams {
     T gamma_inv_cp;  // gamma / cp
     T eta_mu0;       // eta * mu0
     T nu_third;      // nu / 3
+    T nu_third_zeta; // nu / 3 + zeta: the factor of grad(div u) in the momentum equation
     T pT_scale;      // cs2_sound * exp(-lnT0): 1 / (rho T) = pT_scale / (rho cs2)
 };
 
@@ -53,6 +54,7 @@ struct SolveArgs {
     long long fstride;
     Coeffs<T> C;
     PhysParams<T> P;
+    T mxv[3][4];       // (nu / 3 + zeta) C.mx
     T dt;              // used when dt_dev == nullptr
     T alpha, beta;     // alpha_s, beta_s
     int step;          // substep 0, 1, 2

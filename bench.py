@@ -77,7 +77,7 @@ def solve_kernel_name(lib, dev):
     """Which solve kernel the device's (autotuned or pinned) launch shape runs."""
     kind = ctypes.c_int()
     lib.acDeviceGetSolveKernel(dev.handle, ctypes.byref(kind))
-    return {-1: "direct", 0: "delay-line", 1: "sweep"}.get(kind.value, str(kind.value))
+    return {-1: "direct", 0: "delay-line", 1: "sweep", 2: "split"}.get(kind.value, str(kind.value))
 
 
 def run_steps(lib, dev, steps, courant):

@@ -95,7 +95,8 @@ typedef enum {
     AC_solve_tile_y,
     AC_solve_zchunk,
     AC_forcing_period_steps, /* steps between new forcing parameters (config/astaroth.conf:34) */
-    AC_solve_kernel,     /* with a pinned launch shape: 0 = delay-line kernel, 1 = unrolled sweep (FP32) */
+    AC_solve_kernel,     /* with a pinned launch shape: 0 = delay-line kernel, 1 = unrolled sweep (FP32),
+                            2 = role-split kernel; where the shape is autotuned, < 0 leaves the role-split kernel out */
     NUM_INT_PARAMS
 } AcIntParam;
 
