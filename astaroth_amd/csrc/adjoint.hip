@@ -11,6 +11,7 @@
 // halo copy; (C) per output field, the transposed stencils applied to the derivative adjoints
 // by a z-marching kernel, added to lf (first derivatives are antisymmetric, so their transpose
 // is the negative; second, upwind and mixed ones are symmetric).
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 
@@ -279,158 +280,20 @@ __global__ void __launch_bounds__(256) adjoint_param_stage2(const double* ranges
     }
 }
 
-// ---------------------------------------------------------------- adjoint (C), z-marching form
-// The same transposed stencils, organised so that every derivative-adjoint value is read from
-// memory once per use pattern: a thread owns an (x, y) column and walks a chunk of planes. Each
-// output field q has a chain acc[q][k] of partial sums for planes p - 3 + k (k = 0..6), where p
-// is the plane being read. Reading plane p pushes
-//   * its pointwise and in-plane (x / y) contributions into acc[q][3] (plane p itself);
-//   * its z-stencil contributions into acc[q][3 -+ i]: a value a(p) under the transposed first
+// ---------------------------------------------------------------- adjoint (C): transposed stencils
+// A thread owns an (x, y) column and walks a chunk of planes. An output field Q has a chain acc[k] of
+// partial sums for planes p - 3 + k (k = 0..6), where p is the plane being read. Reading plane p pushes
+//   * its pointwise and in-plane (x / y) contributions into acc[3] (plane p itself);
+//   * its z-stencil contributions into acc[3 -+ i]: a value a(p) under the transposed first
 //     derivative lands on plane p - i with -d1_i and on p + i with +d1_i; under second
 //     derivative, upwind and D2z of grad(div) with the symmetric weights;
 //   * the xz / yz mixed parts: D_i G(p) = G(x+i, p) - G(x-i, p) lands on p - i with +c_i and on
 //     p + i with -c_i.
-// Plane p - 3 is then complete (acc[q][0]) and its adjoint update is written.
-template <typename T, bool UPWD, int Q>
-__global__ void __launch_bounds__(256) adjoint_transpose_z_kernel(AdjArgs<T> A, int zchunk)
-{
-    const SolveArgs<T>& a = A.s;
-    const int i = threadIdx.x + blockIdx.x * blockDim.x;
-    const int j = threadIdx.y + blockIdx.y * blockDim.y;
-    const int z0 = blockIdx.z * zchunk;
-    if (i >= a.nx || j >= a.ny)
-        return;
-    const int sy = a.mx;
-    const long long sz = a.sz;
-    const Coeffs<T>& C = a.C;
-    const unsigned colb0 = (unsigned)(((i + R) + sy * (j + R)) * (int)sizeof(T));
-    T acc[7];
-#pragma unroll
-    for (int k = 0; k < 7; ++k)
-        acc[k] = T(0);
-
-    const int np = zchunk + 2 * R;
-    for (int it = 0; it < np; ++it) {
-        const int p = z0 - R + it;  // interior plane index being read (array plane p + R)
-        // uniform bases recomputed per plane from an opaque field stride; 32-bit lane offsets
-        const long long nb = opaque_s64(A.count * (long long)sizeof(T));
-        const unsigned colb = opaque(colb0);
-        const char* const pb = (const char*)A.g + sz * (long long)(p + R) * (long long)sizeof(T);
-        // value of derivative-adjoint field k at offset (dx, dy) from this column in plane p;
-        // the signed neighbour offset is added to the column's byte offset in 32-bit unsigned
-        // arithmetic first (the sum is a valid non-negative offset), then to the base pointer
-        auto ld = [&](int k, int dx, int dy) -> T {
-            const unsigned off = colb + (unsigned)((dx + dy * sy) * (int)sizeof(T));
-            return *(const T*)(pb + k * nb + off);
-        };
-        auto d1x = [&](int k) {
-            return C.d1[0][1] * (ld(k, 1, 0) - ld(k, -1, 0)) + C.d1[0][2] * (ld(k, 2, 0) - ld(k, -2, 0)) +
-                   C.d1[0][3] * (ld(k, 3, 0) - ld(k, -3, 0));
-        };
-        auto d1y = [&](int k) {
-            return C.d1[1][1] * (ld(k, 0, 1) - ld(k, 0, -1)) + C.d1[1][2] * (ld(k, 0, 2) - ld(k, 0, -2)) +
-                   C.d1[1][3] * (ld(k, 0, 3) - ld(k, 0, -3));
-        };
-        // symmetric stencil along x (ax = 0) or y (ax = 1), centre weight included
-        auto sym = [&](int k, int ax, const T* w) {
-            const int ex = ax == 0, ey = ax == 1;
-            return w[0] * ld(k, 0, 0) + w[1] * (ld(k, ex, ey) + ld(k, -ex, -ey)) +
-                   w[2] * (ld(k, 2 * ex, 2 * ey) + ld(k, -2 * ex, -2 * ey)) +
-                   w[3] * (ld(k, 3 * ex, 3 * ey) + ld(k, -3 * ex, -3 * ey));
-        };
-        auto mixed_xy = [&](int k) {
-            T r = T(0);
-#pragma unroll
-            for (int o = 1; o <= 3; ++o)
-                r += C.mx[0][o] * ((ld(k, o, o) + ld(k, -o, -o)) - (ld(k, o, -o) + ld(k, -o, o)));
-            return r;
-        };
-        // transposed first derivative along z of a column value: -d1_o on p - o, +d1_o on p + o
-        auto push_anti = [&](T v) {
-#pragma unroll
-            for (int o = 1; o <= 3; ++o) {
-                acc[3 - o] -= C.d1[2][o] * v;
-                acc[3 + o] += C.d1[2][o] * v;
-            }
-        };
-        auto push_sym = [&](T v, const T* w) {
-            acc[3] += w[0] * v;
-#pragma unroll
-            for (int o = 1; o <= 3; ++o) {
-                acc[3 - o] += w[o] * v;
-                acc[3 + o] += w[o] * v;
-            }
-        };
-        // xz (ax = 0) or yz (ax = 1) mixed part of field k: D_o G(p) on p - o with +c_o, on
-        // p + o with -c_o
-        auto push_mixed = [&](int k, int ax) {
-            const int ex = ax == 0, ey = ax == 1;
-            const T* w = C.mx[ax == 0 ? 1 : 2];
-#pragma unroll
-            for (int o = 1; o <= 3; ++o) {
-                const T D = w[o] * (ld(k, o * ex, o * ey) - ld(k, -o * ex, -o * ey));
-                acc[3 - o] += D;
-                acc[3 + o] -= D;
-            }
-        };
-
-        // own stencils: first derivatives in x / y (absent for d_i A_i), the Laplacian, the
-        // upwind operators (lnrho and u); the z parts pushed into the chain
-        {
-            constexpr int kx = g_index(Q, ROLE_DX), ky = g_index(Q, ROLE_DY);
-            constexpr int kz = g_index(Q, ROLE_DZ), kl = g_index(Q, ROLE_LAP);
-            T r = sym(kl, 0, C.d2[0]) + sym(kl, 1, C.d2[1]);
-            if constexpr (kx >= 0)
-                r -= d1x(kx);
-            if constexpr (ky >= 0)
-                r -= d1y(ky);
-            if constexpr (UPWD && Q < 4)
-                r += sym(g_index(Q, ROLE_UPX), 0, C.up[0]) + sym(g_index(Q, ROLE_UPY), 1, C.up[1]);
-            acc[3] += r;
-            if constexpr (kz >= 0)
-                push_anti(ld(kz, 0, 0));
-            push_sym(ld(kl, 0, 0), C.d2[2]);
-            if constexpr (UPWD && Q < 4)
-                push_sym(ld(g_index(Q, ROLE_UPZ), 0, 0), C.up[2]);
-        }
-        // grad(div v) parts of the vector components (u: Q = 1..3 from G_GDU, A: 4..6 from G_GDA)
-        if (Q >= 1 && Q <= 6) {
-            const int gb = Q <= 3 ? G_GDU : G_GDA;
-            const int comp = (Q - 1) % 3;
-            if (comp == 0) {
-                acc[3] += sym(gb + 0, 0, C.d2[0]) + mixed_xy(gb + 1);
-                push_mixed(gb + 2, 0);  // d_xz of G2
-            }
-            else if (comp == 1) {
-                acc[3] += mixed_xy(gb + 0) + sym(gb + 1, 1, C.d2[1]);
-                push_mixed(gb + 2, 1);  // d_yz of G2
-            }
-            else {
-                push_mixed(gb + 0, 0);  // d_xz of G0
-                push_mixed(gb + 1, 1);  // d_yz of G1
-                push_sym(ld(gb + 2, 0, 0), C.d2[2]);
-            }
-        }
-
-        // ---- plane p - 3 is complete: its adjoint update
-        if (it >= 2 * R) {
-            const long long ob = sz * (long long)p * (long long)sizeof(T);  // array plane p - 3 + R
-            T* lfp = (T*)((char*)A.lf + Q * nb + ob + colb);
-            *lfp = *lfp + a.dt * acc[0];
-        }
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-            acc[k] = acc[k + 1];
-        acc[6] = T(0);
-    }
-}
-
-// ---------------------------------------------------------------- adjoint (C), LDS-staged form
-// The same per-output-field transposes on 64 x 16, 64 x 8 or 64 x 4 column blocks: the
-// derivative-adjoint fields output field Q reads with in-plane (x / y) neighbours are DMA'd
-// plane by plane into LDS (with their radius-3 halo, double-buffered, as the forward solve
-// stages its planes), fields read only at the column come straight from memory, and the z parts
-// use the same push chain.
+// Plane p - 3 is then complete (acc[0]) and its adjoint update is written. The derivative-adjoint
+// fields that Q reads with in-plane (x / y) neighbours are DMA'd plane by plane into LDS with their
+// radius-3 halo, one plane ahead; fields read only at the column come straight from memory. Halos
+// are read from the periodic images, wrapped at any grid size, so the derivative adjoints need no
+// halo fill.
 
 // Fields of output Q that are read with in-plane neighbours ("staged"), in slot order: its own
 // x / y first derivatives (those that exist), Laplacian and, for lnrho and u with upwinding, the
@@ -499,86 +362,94 @@ __host__ __device__ constexpr int column_field(int Q, bool upwd, int slot)
     return (Q <= 3 ? G_GDU : G_GDA) + 2;
 }
 
-// TY = 16 (FP32) or 8 where ny allows (1024- or 512-thread workgroups: the staged in-plane halo
-// drops from 10/4 to 22/16 or 14/8 rows per output row, and FP64 runs two waves per SIMD
-// instead of one), else 4.
-template <typename T, bool UPWD, int Q, int TY>
-__global__ void __launch_bounds__(64 * TY) adjoint_transpose_lds_kernel(AdjArgs<T> A, int zchunk,
-                                                                        int ntx, int nty)
+// Column blocks: 64 x 16 in FP32, else 32 x 16 or 16 x 16, whichever loads the fewest LDS cells for the
+// grid (the radius-3 halo makes that 1.50, 1.63 and 1.89 per output cell).
+constexpr int TY_T = 16;
+template <typename T, int TX>
+struct TransposeTile {
+    static constexpr int LX = TX + 2 * R, LY = TY_T + 2 * R;
+    static constexpr int NW = TX * TY_T / 64;
+    static constexpr int WPE = (int)sizeof(T) / 4;
+    static constexpr int LPW = LX * LY * WPE;
+    static constexpr int NR = ((LPW + 63) / 64 + NW - 1) / NW;
+    static constexpr int LPS = NR * NW * 64 / WPE;  // padded field-plane stride in LDS (elements)
+};
+constexpr int most_staged(bool upwd) { return upwd ? 8 : 6; }
+
+// This wave's memory operations and LDS reads are done, then the workgroup barrier.
+__device__ __forceinline__ void transpose_barrier()
 {
-    constexpr int TX = 64;
-    constexpr int LX = TX + 2 * R, LY = TY + 2 * R;
-    constexpr int LP = LX * LY;
-    constexpr int NT = TX * TY, NW = NT / 64;
-    constexpr int WPE = (int)sizeof(T) / 4;
-    constexpr int LPW = LP * WPE;
-    constexpr int NCHUNK = (LPW + 63) / 64;
-    constexpr int NR = (NCHUNK + NW - 1) / NW;
-    constexpr int LPS = NR * NW * 64 / WPE;  // padded field-plane stride in LDS (elements)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ int wrap_index(int i, int n)
+{
+    while (i < 0)
+        i += n;
+    while (i >= n)
+        i -= n;
+    return i;
+}
+
+// Output field Q over one column block and z-chunk [z0, z1). lds0 and lds1 are two arrays, named
+// statically by the two plane steps of an iteration: LDS reads of one then need not wait for the DMA
+// into the other.
+template <typename T, bool UPWD, int Q, int TX>
+__device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T* lds1, int x0, int y0,
+                                                int z0, int z1)
+{
+    using G = TransposeTile<T, TX>;
+    constexpr int LX = G::LX, LPS = G::LPS, NR = G::NR, NW = G::NW, WPE = G::WPE;
     constexpr int NS = staged_count(Q, UPWD);
     constexpr int NC = column_count(Q, UPWD);
-    __shared__ T lds[2][NS * LPS];
-
+    static_assert(NS <= most_staged(UPWD), "LDS planes");
     const SolveArgs<T>& a = A.s;
-    // XCD-aware numbering: consecutive hardware block ids go to different XCDs, so each XCD is
-    // handed a contiguous range of tiles (whose y neighbours then share its L2)
-    const int nblocks = (int)gridDim.x;
-    int bid = (int)blockIdx.x;
-    if ((nblocks & 7) == 0)
-        bid = (bid & 7) * (nblocks >> 3) + (bid >> 3);
-    const int tile_x = bid % ntx;
-    const int rest = bid / ntx;
-    const int tile_y = rest % nty;
-    const int chunk = rest / nty;
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int tid = tx + TX * ty;
-    // wave-uniform: a scalar register in FP32 (scalar M0 arithmetic for the DMA); FP64 keeps
-    // the vector form, as the forward kernels do
-    const int wave = sizeof(T) == 4 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    const int tid = threadIdx.x;
+    const int tx = tid % TX, ty = tid / TX;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int x0 = tile_x * TX, y0 = tile_y * TY, z0 = chunk * zchunk;
     const int sy = a.mx;
     const long long sz = a.sz;
     const Coeffs<T>& C = a.C;
+    const bool inside = x0 + tx < a.nx && y0 + ty < a.ny;
 
-    // DMA: every lane moves one dword per chunk; padding lanes re-read dword 0 of the plane.
-    // The x / y halo of a tile is read from the periodic images inside the interior, so the
-    // derivative adjoints need no halo fill.
+    // DMA: every lane moves one dword per round; padding lanes re-read dword 0 of the plane
     unsigned g_off[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
         int d = (wave + r * NW) * 64 + lane;
-        if (d >= LPW)
+        if (d >= G::LPW)
             d = 0;
         const int e = d / WPE, wd = d - e * WPE;
         const int ly = e / LX, lx = e - ly * LX;
-        int gx = x0 + lx - R, gy = y0 + ly - R;
-        gx += gx < 0 ? a.nx : (gx >= a.nx ? -a.nx : 0);
-        gy += gy < 0 ? a.ny : (gy >= a.ny ? -a.ny : 0);
+        const int gx = wrap_index(x0 + lx - R, a.nx), gy = wrap_index(y0 + ly - R, a.ny);
         g_off[r] = (unsigned)(((gx + R) + sy * (gy + R)) * (int)sizeof(T) + 4 * wd);
     }
     // byte offset of interior plane p (z wrapped periodically) within a field
     auto plane_b = [&](int p) {
-        p += p < 0 ? a.nz : (p >= a.nz ? -a.nz : 0);
-        return sz * (long long)(p + R) * (long long)sizeof(T);
+        return sz * (long long)(wrap_index(p, a.nz) + R) * (long long)sizeof(T);
     };
-    auto dma_plane = [&](int p, int b, long long nb) {
+    auto dma_plane = [&](int p, T* dst, long long nb) {
         const char* pb = (const char*)A.g + plane_b(p);
+        const int first = opaque_s32(wave * (64 / WPE));
 #pragma unroll
         for (int sl = 0; sl < NS; ++sl) {
             const char* src = pb + staged_field(Q, UPWD, sl) * nb;
-            char* dst = (char*)&lds[b][sl * LPS];
 #pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const int j = wave + r * NW;
+            for (int r = 0; r < NR; ++r)
                 __builtin_amdgcn_global_load_lds((const void*)(src + opaque(g_off[r])),
-                                                 (lds_ptr_t)(dst + 256 * j), 4, 0, 0);
-            }
+                                                 (lds_ptr_t)(dst + sl * LPS + first + r * NW * (64 / WPE)),
+                                                 4, 0, 0);
         }
     };
 
     const int ctr = (ty + R) * LX + (tx + R);
-    const unsigned colb0 = (unsigned)(((x0 + tx + R) + sy * (y0 + ty + R)) * (int)sizeof(T));
+    // columns past the grid read a column inside it and write nothing
+    const unsigned colb0 = (unsigned)((((inside ? x0 + tx : 0) + R) + sy * ((inside ? y0 + ty : 0) + R)) *
+                                      (int)sizeof(T));
     T acc[7];
 #pragma unroll
     for (int k = 0; k < 7; ++k)
@@ -587,7 +458,7 @@ __global__ void __launch_bounds__(64 * TY) adjoint_transpose_lds_kernel(AdjArgs<
     T col[NC], coln[NC];
     // lambda_f of the plane completed in this step (lfc) and in the next one (loaded a plane
     // ahead); the local stage has already added its pointwise part
-    T lfc = T(0), lfn = T(0);
+    T lfc = T(0), lfn = T(0), done = T(0);
     auto load_cols = [&](int p, long long nb, unsigned colb, T* dst) {
         const char* pb = (const char*)A.g + plane_b(p);
 #pragma unroll
@@ -601,27 +472,26 @@ __global__ void __launch_bounds__(64 * TY) adjoint_transpose_lds_kernel(AdjArgs<
 
     {
         const long long nb = A.count * (long long)sizeof(T);
-        dma_plane(z0 - R, 0, nb);
+        dma_plane(z0 - R, lds0, nb);
         load_cols(z0 - R, nb, colb0, col);
     }
-    plane_barrier();
-    const int np = zchunk + 2 * R;
-    for (int it = 0; it < np; ++it) {
+    transpose_barrier();
+    const int np = z1 - z0 + 2 * R;
+    auto step = [&](int it, const T* lds, T* next) {
         const int p = z0 - R + it;
-        const int cur = it & 1;
         const long long nb = opaque_s64(A.count * (long long)sizeof(T));
         const unsigned colb = opaque(colb0);
         if (it + 1 < np) {
-            dma_plane(p + 1, cur ^ 1, nb);
+            dma_plane(p + 1, next, nb);
             load_cols(p + 1, nb, colb, coln);
-            if (it + 1 >= 2 * R) {
-                const long long ob = out_off(it + 1, nb, colb);
-                lfn = *(const T*)((const char*)A.lf + ob);
-            }
+            if (it + 1 >= 2 * R)
+                lfn = *(const T*)((const char*)A.lf + out_off(it + 1, nb, colb));
         }
-        auto lds_at = [&](int sl, int dx, int dy) -> T {
-            return lds[cur][sl * LPS + ctr + dy * LX + dx];
-        };
+        // the plane completed in the last step: stored here and not before the barrier, which waits for
+        // every store
+        if (it > 2 * R && inside)
+            *(T*)((char*)A.lf + out_off(it - 1, nb, colb)) = done;
+        auto lds_at = [&](int sl, int dx, int dy) -> T { return lds[sl * LPS + ctr + dy * LX + dx]; };
         auto d1x = [&](int sl) {
             return C.d1[0][1] * (lds_at(sl, 1, 0) - lds_at(sl, -1, 0)) +
                    C.d1[0][2] * (lds_at(sl, 2, 0) - lds_at(sl, -2, 0)) +
@@ -712,10 +582,8 @@ __global__ void __launch_bounds__(64 * TY) adjoint_transpose_lds_kernel(AdjArgs<
             }
         }
 
-        if (it >= 2 * R) {
-            const long long ob = out_off(it, nb, colb);
-            *(T*)((char*)A.lf + ob) = lfc + a.dt * acc[0];
-        }
+        if (it >= 2 * R)
+            done = lfc + a.dt * acc[0];
 #pragma unroll
         for (int k = 0; k < 6; ++k)
             acc[k] = acc[k + 1];
@@ -725,7 +593,52 @@ __global__ void __launch_bounds__(64 * TY) adjoint_transpose_lds_kernel(AdjArgs<
             col[c] = coln[c];
         lfc = lfn;
         // plane p + 1 has landed and every wave is done with this one
-        plane_barrier();
+        transpose_barrier();
+    };
+    for (int it = 0; it < np; it += 2) {
+        step(it, lds0, lds1);
+        if (it + 1 < np)
+            step(it + 1, lds1, lds0);
+    }
+    if (inside)
+        *(T*)((char*)A.lf + out_off(np - 1, A.count * (long long)sizeof(T), colb0)) = done;
+}
+
+// All output fields in one launch: a workgroup takes one field of one column block and z-chunk. One
+// field has 64 workgroups at 128^3 (64 x 16 columns, 32 planes), a quarter of the CUs; eight launches of
+// them took 649 us FP32, this one 240, with 47 + 16 fields read or written at least once (530 MB). From
+// 256^3 on, where one field fills the chip, both are bound by the memory (1.55 ms). On grids that 64
+// columns do not divide, an unstaged kernel per field and a halo fill of the derivative adjoints took
+// 0.85 ms (72 x 60 x 50 FP64); this takes 60 us. The fields of one block follow each other (all blocks of
+// one field first) since neighbouring blocks in step share more than the fields of a block do (256^3
+// FP32, whole adjoint substep: 2.93 ms against 3.24 with the fields of a block side by side).
+template <typename T, bool UPWD, int TX>
+__global__ void __launch_bounds__(TX * TY_T) adjoint_transpose_kernel(AdjArgs<T> A, int zchunk, int ntx,
+                                                                      int nty, int nq)
+{
+    using G = TransposeTile<T, TX>;
+    __shared__ T lds0[most_staged(UPWD) * G::LPS];
+    __shared__ T lds1[most_staged(UPWD) * G::LPS];
+    // Consecutive hardware block ids go to different XCDs, so each XCD is handed a contiguous range
+    // of blocks, whose y neighbours and whose other fields then share its L2.
+    const int ntiles = ntx * nty * ((A.s.nz + zchunk - 1) / zchunk);
+    const int per_xcd = (ntiles + 7) >> 3;
+    const int slot = (int)blockIdx.x >> 3;
+    const int t = ((int)blockIdx.x & 7) * per_xcd + slot % per_xcd;
+    if (t >= ntiles)
+        return;
+    const int x0 = t % ntx * TX, y0 = t / ntx % nty * TY_T, z0 = t / (ntx * nty) * zchunk;
+    const int z1 = min(z0 + zchunk, A.s.nz);
+    // the fields with the most to read first; ss last, which a run without entropy leaves out
+    switch (slot / per_xcd) {
+    case 0: transpose_block<T, UPWD, 1, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 1: transpose_block<T, UPWD, 2, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 2: transpose_block<T, UPWD, 3, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 3: transpose_block<T, UPWD, 4, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 4: transpose_block<T, UPWD, 5, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 5: transpose_block<T, UPWD, 6, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    case 6: transpose_block<T, UPWD, 0, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
+    default: transpose_block<T, UPWD, 7, TX>(A, lds0, lds1, x0, y0, z0, z1); break;
     }
 }
 
@@ -749,6 +662,40 @@ void launch_tangent(const AdjArgs<T>& A, bool upwd, bool entropy, hipStream_t s)
 long long adjoint_num_blocks(int nx, int ny, int nz)
 {
     return (long long)((nx + 63) / 64) * ((ny + 3) / 4) * nz;
+}
+
+struct TransposeShape {
+    int tx, zchunk;
+};
+
+// The column block that loads the fewest cells, the wider of equals; then the z-chunk with the least of
+// plane steps (six of them start a chunk up) over all workgroups per CU plus half of one workgroup's,
+// which the last ones to finish leave the chip idle for.
+static TransposeShape transpose_shape(int realsize, int nx, int ny, int nz, int nq)
+{
+    TransposeShape best{16, nz};
+    long long least = 1ll << 62;
+    for (int tx : {64, 32, 16}) {
+        const long long cells = (long long)((nx + tx - 1) / tx) * (tx + 2 * R);
+        if (cells < least && !(tx == 64 && realsize == 8)) {
+            least = cells;
+            best.tx = tx;
+        }
+    }
+    // workgroups per CU: LDS holds one of 64 x 16 FP32 and 32 x 16 FP64, two of half their size
+    const int per_cu = best.tx * realsize >= 256 ? 1 : (best.tx * realsize >= 128 ? 2 : 4);
+    const long long tiles = (long long)((nx + best.tx - 1) / best.tx) * ((ny + TY_T - 1) / TY_T);
+    double cost = 1e30;
+    for (int nch = 1; nch <= nz; ++nch) {
+        const int zc = (nz + nch - 1) / nch;
+        const double groups = (double)(tiles * ((nz + zc - 1) / zc) * nq) / (256.0 * per_cu);
+        const double c = (std::max(groups, 1.0) + 0.5) * (zc + 2 * R);
+        if (c < cost) {
+            cost = c;
+            best.zchunk = zc;
+        }
+    }
+    return best;
 }
 
 template <typename T>
@@ -776,66 +723,27 @@ void launch_adjoint(const AdjArgs<T>& A, bool upwd, bool entropy, double* param_
                        (const double*)A.partials, nb, ranges);
     hipLaunchKernelGGL(adjoint_param_stage2, dim3(1), dim3(256), 0, s, (const double*)ranges,
                        param_grad);
-    // (C) transposed stencils, z-marching over chunks of planes: the LDS-staged form where the
-    // grid fits its 64 x 4 column blocks (it reads the periodic images itself), else the plain
-    // form after (B) a periodic fill of the derivative adjoints
-    const bool staged = A.s.nx % 64 == 0 && A.s.ny % 4 == 0 && A.s.nz >= R;
-    for (int k0 = 0; !staged && k0 < NG; k0 += NF) {
-        T* ptrs[NF];
-        const int cnt = NG - k0 < NF ? NG - k0 : NF;
-        for (int q = 0; q < cnt; ++q)
-            ptrs[q] = A.g + (long long)(k0 + q) * A.count;
-        launch_periodic_fill<T>(ptrs, cnt, A.s.nx, A.s.ny, A.s.nz, s);
-    }
-    // the transposes' column-block height: 16 (FP32) or 8 where ny allows, else 4
-    constexpr int TYB = sizeof(T) == 4 ? 16 : 8;
-    const int tyc = A.s.ny % TYB == 0 ? TYB : (A.s.ny % 8 == 0 ? 8 : 4);
-    const int ntx = A.s.nx / 64, nty = A.s.ny / tyc;
-    // z-chunks: 64 planes where that still gives the staged form at least 256 workgroups (one
-    // per CU; 256^3: 9.20 -> 9.03 ms per adjoint step against 32-plane chunks), else the largest
-    // of 32, 16 and 8 below nz
-    int zc = A.s.nz;
-    if (staged && A.s.nz % 64 == 0 && A.s.nz > 64 && (long long)ntx * nty * (A.s.nz / 64) >= 256) {
-        zc = 64;
-    }
-    else {
-        for (int cand : {32, 16, 8})
-            if (A.s.nz % cand == 0 && A.s.nz > cand) {
-                zc = cand;
-                break;
-            }
-    }
-    const dim3 bpz(bpg.x, bpg.y, (unsigned)(A.s.nz / zc));
-    const dim3 bps((unsigned)(ntx * nty * (A.s.nz / zc)), 1, 1), tpbb(64, TYB, 1), tpb8(64, 8, 1);
-#define AC_ADJ_Q(Q)                                                                                \
+    // (C) transposed stencils. Without the entropy equation ss is not evolved (f'_7 = f_7): its lambda_f
+    // passes through and the local stage has set its lambda_w to alpha * 0.
+    const int nq = entropy ? NF : NF - 1;
+    const TransposeShape sh = transpose_shape((int)sizeof(T), A.s.nx, A.s.ny, A.s.nz, nq);
+    const int ntx = (A.s.nx + sh.tx - 1) / sh.tx, nty = (A.s.ny + TY_T - 1) / TY_T;
+    const int ntiles = ntx * nty * ((A.s.nz + sh.zchunk - 1) / sh.zchunk);
+    const dim3 grid((unsigned)((ntiles + 7) / 8 * 8 * nq)), block(sh.tx * TY_T);
+#define AC_TRANSPOSE(TX)                                                                           \
     do {                                                                                           \
-        if (staged && tyc == TYB) {                                                                \
-            if (upwd) hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, true, Q, TYB>), bps, tpbb, 0, s, A, zc, ntx, nty); \
-            else hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, false, Q, TYB>), bps, tpbb, 0, s, A, zc, ntx, nty);    \
-        }                                                                                          \
-        else if (staged && tyc == 8) {                                                             \
-            if (upwd) hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, true, Q, 8>), bps, tpb8, 0, s, A, zc, ntx, nty); \
-            else hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, false, Q, 8>), bps, tpb8, 0, s, A, zc, ntx, nty);    \
-        }                                                                                          \
-        else if (staged) {                                                                         \
-            if (upwd) hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, true, Q, 4>), bps, tpb, 0, s, A, zc, ntx, nty); \
-            else hipLaunchKernelGGL((adjoint_transpose_lds_kernel<T, false, Q, 4>), bps, tpb, 0, s, A, zc, ntx, nty);    \
-        }                                                                                          \
-        else if (upwd) hipLaunchKernelGGL((adjoint_transpose_z_kernel<T, true, Q>), bpz, tpb, 0, s, A, zc); \
-        else hipLaunchKernelGGL((adjoint_transpose_z_kernel<T, false, Q>), bpz, tpb, 0, s, A, zc);    \
+        if (upwd) hipLaunchKernelGGL((adjoint_transpose_kernel<T, true, TX>), grid, block, 0, s, A, sh.zchunk, ntx, nty, nq); \
+        else hipLaunchKernelGGL((adjoint_transpose_kernel<T, false, TX>), grid, block, 0, s, A, sh.zchunk, ntx, nty, nq);     \
     } while (0)
-    AC_ADJ_Q(0);
-    AC_ADJ_Q(1);
-    AC_ADJ_Q(2);
-    AC_ADJ_Q(3);
-    AC_ADJ_Q(4);
-    AC_ADJ_Q(5);
-    AC_ADJ_Q(6);
-    // without the entropy equation ss is not evolved (f'_7 = f_7): its lambda_f passes through
-    // and the local stage has set its lambda_w to alpha * 0
-    if (entropy)
-        AC_ADJ_Q(7);
-#undef AC_ADJ_Q
+    if (sh.tx == 16)
+        AC_TRANSPOSE(16);
+    else if (sh.tx == 32)
+        AC_TRANSPOSE(32);
+#if !AC_DOUBLE_PRECISION
+    else
+        AC_TRANSPOSE(64);
+#endif
+#undef AC_TRANSPOSE
 #undef AC_ADJ
 }
 

@@ -110,6 +110,12 @@ __device__ __forceinline__ unsigned opaque(unsigned v)
     asm volatile("" : "+v"(v));
     return v;
 }
+// The same for a wave-uniform value (a scalar register).
+__device__ __forceinline__ int opaque_s32(int v)
+{
+    asm volatile("" : "+s"(v));
+    return v;
+}
 // The same for a wave-uniform 64-bit value kept in a scalar register pair: recomputing
 // per-field bases from it each plane step beats holding eight bases per array across the loop.
 __device__ __forceinline__ long long opaque_s64(long long v)

@@ -133,11 +133,6 @@ __device__ __forceinline__ const S* step_args()
     typedef const __attribute__((address_space(4))) S karg;
     return (const S*)(karg*)opaque_s64((long long)__builtin_amdgcn_kernarg_segment_ptr());
 }
-__device__ __forceinline__ int opaque_s32(int v)
-{
-    asm volatile("" : "+s"(v));
-    return v;
-}
 
 template <int V>
 struct IntC {

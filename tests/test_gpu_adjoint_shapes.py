@@ -1,0 +1,31 @@
+"""The adjoint's transposed stencils on grids their column blocks do not divide: one column, row or
+plane past a block, grids narrower than a block and as narrow as the stencil, and ragged last z-chunks.
+The tangent substep (one cell per thread) is the reference: <T(dx), y> = <dx, A(y)>, to the rounding of
+the sums in each precision, as for the grids that the blocks divide; and repeated runs agree bit for bit."""
+import os
+import sys
+
+import pytest
+
+from astaroth_amd import astaroth as ac
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+from test_gpu_adjoint import initial, physics_info, say, substep_dot_product  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", params=["fp64", "fp32"])
+def lib(request, require_gpu):
+    return ac.load(request.param)
+
+
+@pytest.mark.parametrize("n", [(65, 17, 9), (33, 15, 7), (17, 33, 70), (31, 16, 5), (5, 4, 3), (128, 48, 67)])
+@pytest.mark.parametrize("upwd,entropy,step", [(True, True, 0), (False, True, 1), (True, False, 2)])
+def test_transposes_on_any_grid(lib, n, upwd, entropy, step):
+    say(f"case adjoint shapes {lib.precision} n={n} upwd={upwd} entropy={entropy} step={step}")
+    info = physics_info(lib, n, AC_lupwd=upwd, AC_lentropy=entropy)
+    f = initial(lib, info, 3 + step)
+    runs = [substep_dot_product(lib, info, f, step, entropy, 7 + step) for _ in range(2)]
+    assert runs[0][2] < (1e-12 if lib.precision == "fp64" else 1e-5)
+    assert runs[0][:3] == runs[1][:3] and bool((runs[0][3] == runs[1][3]).all())
