@@ -1059,24 +1059,27 @@ AcResult acDeviceGetTimestep(const Device d, const Stream stream, double* dt)
     return AC_SUCCESS;
 }
 
-AcResult acDeviceIntegrateSubstepDeviceDt(const Device d, const Stream stream,
-                                          const int step_number, const AcReal courant)
+// One substep with the device-resident timestep. The pair of maxima that substep 2 reduces into is
+// cleared before it: by substep 0 of the same step where a call runs whole steps with the role-split
+// kernel (`clear` says so at substep 0, and comes back at substep 2), else by a launch of its own;
+// the accumulated time of the call likewise at its first step.
+static AcResult substep_device_dt(Device d, hipStream_t s, const int step_number, const AcReal courant,
+                                  const bool clear, const bool clear_time)
 {
-    if (step_number < 0 || step_number > 2)
-        return fail("acDeviceIntegrateSubstepDeviceDt: step_number must be 0, 1 or 2");
-    AC_HIP_CHECK(hipSetDevice(d->id));
-    hipStream_t s = get_stream(d, stream);
-    if (ensure_shape(d, s, step_number == 0) != AC_SUCCESS)
-        return AC_FAILURE;
     SolveArgs<AcReal> a;
     fill_solve_args(d, a, step_number, (AcReal)0);
     if (d->cfl_mode == 0)
         a.cfl_cdt = (double)courant;
     a.umax2_cur = (const double*)(d->umax2 + 2 * d->cfl_cur);
     const int nxt = 1 - d->cfl_cur;
+    unsigned long long* next = d->umax2 + 2 * nxt;
+    if (step_number == 0 && clear) {
+        a.umax2_next = next;
+        a.time_acc = clear_time ? d->time_acc : nullptr;
+    }
     if (step_number == 2) {
-        unsigned long long* next = d->umax2 + 2 * nxt;
-        launch_zero_bytes(next, 2 * sizeof(unsigned long long), s);
+        if (!clear)
+            launch_zero_bytes(next, 2 * sizeof(unsigned long long), s);
         a.time_acc = d->time_acc;
         if (d->cfl_mode == 0) {
             // max |u_new|^2, reduced by the solve kernel itself (by the forcing kernel when
@@ -1096,11 +1099,23 @@ AcResult acDeviceIntegrateSubstepDeviceDt(const Device d, const Stream stream,
     }
     const AcResult r = launch_solve(d, a, s);
     if (r == AC_SUCCESS && step_number == 2 && forcing_on(d))
-        launch_forcing_step(d, a, s, d->cfl_mode == 0 ? d->umax2 + 2 * nxt : nullptr);
+        launch_forcing_step(d, a, s, d->cfl_mode == 0 ? next : nullptr);
     if (step_number == 2)
         d->cfl_cur = nxt;
     d->cfl_courant = (double)courant;
     return r;
+}
+
+AcResult acDeviceIntegrateSubstepDeviceDt(const Device d, const Stream stream,
+                                          const int step_number, const AcReal courant)
+{
+    if (step_number < 0 || step_number > 2)
+        return fail("acDeviceIntegrateSubstepDeviceDt: step_number must be 0, 1 or 2");
+    AC_HIP_CHECK(hipSetDevice(d->id));
+    hipStream_t s = get_stream(d, stream);
+    if (ensure_shape(d, s, step_number == 0) != AC_SUCCESS)
+        return AC_FAILURE;
+    return substep_device_dt(d, s, step_number, courant, false, false);
 }
 
 AcResult acDeviceIntegrateStepsCFL(const Device d, const Stream stream, const int nsteps,
@@ -1109,17 +1124,28 @@ AcResult acDeviceIntegrateStepsCFL(const Device d, const Stream stream, const in
     AC_HIP_CHECK(hipSetDevice(d->id));
     hipStream_t s = get_stream(d, stream);
     const int3 n = d->local_config.int3_params[AC_nlocal];
-    // time_acc accumulates the simulated time of this call (the forcing's step start times are
-    // AC_current_time plus it)
-    launch_zero_bytes(d->time_acc, sizeof(double), s);
     // The tiled solve kernels read the periodic images of the halo cells themselves, so no fill
     // precedes their substeps (launch_solve fills first where another kernel runs). The reference
     // timestep modes reduce over the state entering substep 2 with derivatives that read the
-    // halos: that substep keeps its fill. One fill up front also gives the launch autotuner
-    // (first substep on a new grid) a state with consistent halos.
-    launch_periodic_fill<AcReal>(d->in, NF, n.x, n.y, n.z, s);
+    // halos: that substep keeps its fill. One fill up front gives the launch autotuner (first
+    // substep on a new grid) a state with consistent halos.
+    if (!d->shape_tuned || nsteps <= 0)
+        launch_periodic_fill<AcReal>(d->in, NF, n.x, n.y, n.z, s);
     if (ensure_shape(d, s, nsteps > 0) != AC_SUCCESS)
         return AC_FAILURE;
+    // The role-split kernel clears the maxima and the time itself: three launches a step, where the
+    // up-front fill and the launches that cleared 8 and 16 bytes made six (32^3 FP32, calls of one step:
+    // 22 -> 15 us a step with three states in turn, 40 -> 34 with one).
+    bool clear = false;
+    if (d->shape.tx > 0 && d->shape.kind == 2) {
+        SolveArgs<AcReal> a;
+        fill_solve_args(d, a, 0, (AcReal)0);
+        clear = shape_reads_periodic(a, d->kahan_bits, d->shape);
+    }
+    // time_acc accumulates the simulated time of this call (the forcing's step start times are
+    // AC_current_time plus it)
+    if (!clear || nsteps <= 0)
+        launch_zero_bytes(d->time_acc, sizeof(double), s);
     for (int step = 0; step < nsteps; ++step) {
         for (int sub = 0; sub < 3; ++sub) {
             const bool fused = d->cfl_mode == 0 || sub != 2;
@@ -1127,7 +1153,7 @@ AcResult acDeviceIntegrateStepsCFL(const Device d, const Stream stream, const in
                 launch_periodic_fill<AcReal>(d->in, NF, n.x, n.y, n.z, s);
             d->periodic_fused = fused;
             d->forcing_time_acc = true;
-            const AcResult r = acDeviceIntegrateSubstepDeviceDt(d, stream, sub, courant);
+            const AcResult r = substep_device_dt(d, s, sub, courant, clear, step == 0);
             d->periodic_fused = false;
             d->forcing_time_acc = false;
             if (r != AC_SUCCESS)
@@ -1356,10 +1382,10 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
     // Candidates: the role-split shapes (any grid); in FP32 also the delay-line shapes of 64 x 4 columns
     // that give each CU its two workgroups, which are faster once the state is far larger than the caches
     // (256^3 plain: 0.54 against 0.59 ms per launch; smaller grids 0.105 against 0.079 ms at 128^3, and
-    // FP64 1.59 against 1.36 ms at 256^3); and the direct kernel up to 32^3 cells, where it is about as
-    // fast as the others (32^3 FP32: 0.0092 ms each). Where the configuration leaves the role-split
-    // kernel out: the direct kernel, the delay-line and the sweep shapes of 64 columns. The ring shapes
-    // read halos as stored and never win; they stay pinnable.
+    // FP64 1.59 against 1.36 ms at 256^3). The direct kernel, at most as fast even at 16^3 to 32^3 (32^3 FP32:
+    // 0.0092 ms each) and in need of a fill before each substep (22 against 33 us a step there), is tried
+    // where the configuration leaves the role-split kernel out, with the delay-line and the sweep shapes of
+    // 64 columns. The ring shapes read halos as stored and never win; they stay pinnable.
     std::vector<TiledShape> cands;
     TiledShape split[4];
     const int nsplit = one_slab && !column_kernels_only(d) ? split_candidates(n.x, n.y, n.z, split, 4) : 0;
@@ -1376,7 +1402,7 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
         for (const TiledShape& sh : kSweepShapes)
             if (shape_fits(sh, n) && sweep_applies<AcReal>(ta[0], kb, sh))
                 cands.push_back(sh);
-    if (nsplit == 0 || (long long)n.x * n.y * n.z <= 32768)
+    if (nsplit == 0)
         cands.push_back(TiledShape{0, 0, 0, 0});
     if (cands.size() == 1) {
         d->shape = cands[0];

@@ -62,8 +62,9 @@ struct SolveArgs {
     // pair (x, y) of reduced maxima (double bits); what they hold and the dt formula depend on
     // cfl_mode (see cfl_cell / solve_dt).
     const double* umax2_cur;
-    unsigned long long* umax2_next;  // step 2: atomic max of the pair of the state reduced
-    double* time_acc;                // step 2: accumulated simulated time
+    // step 2: atomic max of the pair of the state reduced; step 0 of the role-split kernel clears it
+    unsigned long long* umax2_next;
+    double* time_acc;                // step 2: accumulated simulated time; step 0 clears it likewise
     double cfl_cdt, cfl_dsmin, cfl_cs;
     int cfl_mode;                    // 0 courant, 1 reference, 2 reference additive
     double cfl_cs2, cfl_cdtv, cfl_visc;  // cs^2, cdtv, max(nu, eta[, gamma chi])

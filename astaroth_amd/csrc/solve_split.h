@@ -182,6 +182,13 @@ __global__ void __launch_bounds__(2 * TX* TY, (sizeof(T) == 4 ? 2 : 1))
     const int tile_y = rest % nty;
     const int chunk = rest / nty;
 
+    if (STEP == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+        // the maxima that substep 2 of this step reduces into, and the call's time at its first step
+        if (a.umax2_next != nullptr)
+            a.umax2_next[0] = a.umax2_next[1] = 0;
+        if (a.time_acc != nullptr)
+            *a.time_acc = 0.0;
+    }
     const int wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int role = wave_all >= NW ? 1 : 0;
     const int wave = wave_all - role * NW;
