@@ -8,6 +8,7 @@
 // Reductions: ref src/core/kernels/reductions.cu:98-219 (map kernel into an n^3 scratchpad, then
 // hipcub DeviceReduce). Here the map is fused into a single pass with FP64 accumulation and a
 // deterministic two-stage tree (fixed grid, fixed order).
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -118,51 +119,73 @@ __device__ __forceinline__ double red_combine(int op, double a, double b)
     return op == 1 ? fmin(a, b) : (op == 2 ? fmax(a, b) : a + b);
 }
 
+// The mapped value of one cell from the values of its arrays, and how many of them a map reads.
 template <typename T>
-__device__ __forceinline__ double red_map(int map, const T* const* bufs, long long c)
+__device__ __forceinline__ double red_map(int map, const T* v)
 {
     switch (map) {
-    case 1: return (double)bufs[0][c];
-    case 2: { const double v = bufs[0][c]; return v * v; }
-    case 3: { const double e = exp((double)bufs[0][c]); return e * e; }
+    case 1: return (double)v[0];
+    case 2: { const double x = v[0]; return x * x; }
+    case 3: { const double e = exp((double)v[0]); return e * e; }
     case 4: {
-        const double x = bufs[0][c], y = bufs[1][c], z = bufs[2][c];
+        const double x = v[0], y = v[1], z = v[2];
         return sqrt(x * x + y * y + z * z);
     }
     case 5: {
-        const double x = bufs[0][c], y = bufs[1][c], z = bufs[2][c];
+        const double x = v[0], y = v[1], z = v[2];
         return x * x + y * y + z * z;
     }
     case 6: {
-        const double x = exp((double)bufs[0][c]), y = exp((double)bufs[1][c]),
-                     z = exp((double)bufs[2][c]);
+        const double x = exp((double)v[0]), y = exp((double)v[1]),
+                     z = exp((double)v[2]);
         return x * x + y * y + z * z;
     }
     case 7: {
-        const double x = bufs[0][c], y = bufs[1][c], z = bufs[2][c];
-        return sqrt(x * x + y * y + z * z) / sqrt(exp((double)bufs[3][c]));
+        const double x = v[0], y = v[1], z = v[2];
+        return sqrt(x * x + y * y + z * z) / sqrt(exp((double)v[3]));
     }
     case 8: {
-        const double x = bufs[0][c], y = bufs[1][c], z = bufs[2][c];
-        return (x * x + y * y + z * z) / exp((double)bufs[3][c]);
+        const double x = v[0], y = v[1], z = v[2];
+        return (x * x + y * y + z * z) / exp((double)v[3]);
     }
     default: return 0.0;
     }
 }
+static int red_arrays(int map) { return map < 1 || map > 8 ? 0 : (map <= 3 ? 1 : (map <= 6 ? 3 : 4)); }
 
-// Interior cell number t (x fastest) -> index in an m^3 array, in the index type I: 32-bit
-// unsigned when the interior has fewer than 2^31 cells and the array fewer than 2^32 (every grid
-// up to about 1600^3; use_index32 below), 64-bit otherwise. The grid-stride loops visit the same
-// cells in the same order with either type, so the reductions are bit-identical.
+// The interior cells t, t + step, t + 2 step, ... (x fastest) as indices in an m^3 array. The two
+// divisions of each number are taken once, and the steps add (di, dj, dk) with carries. I is 32-bit
+// unsigned when the interior has fewer than 2^31 cells and the array fewer than 2^32 (every grid up
+// to about 1600^3; use_index32 below), 64-bit otherwise; either visits the same cells in the same order.
 template <typename I>
-__device__ __forceinline__ I interior_index(I t, I nx, I ny, I mx, I sz)
-{
-    const I i = t % nx;
-    const I r = t / nx;
-    const I j = r % ny;
-    const I k = r / ny;
-    return (i + R) + mx * (j + R) + sz * (k + R);
-}
+struct CellWalk {
+    I i, j, k, di, dj, dk, nx, ny, mx, sz;
+    __device__ __forceinline__ CellWalk(I t, I step, int nx_, int ny_, int mx_, int my_)
+        : nx((I)nx_), ny((I)ny_), mx((I)mx_), sz((I)mx_ * (I)my_)
+    {
+        i = t % nx;
+        j = t / nx % ny;
+        k = t / nx / ny;
+        di = step % nx;
+        dj = step / nx % ny;
+        dk = step / nx / ny;
+    }
+    __device__ __forceinline__ I cell() const { return (i + R) + mx * (j + R) + sz * (k + R); }
+    __device__ __forceinline__ void advance()
+    {
+        i += di;
+        j += dj;
+        k += dk;
+        if (i >= nx) {
+            i -= nx;
+            ++j;
+        }
+        if (j >= ny) {
+            j -= ny;
+            ++k;
+        }
+    }
+};
 
 static bool use_index32(int nx, int ny, int nz)
 {
@@ -257,16 +280,37 @@ __device__ __forceinline__ double block_reduce(int op, double v, double* sh)
     return r;
 }
 
-template <typename T, typename I>
+// NA arrays are read. The values of eight (one array) or four cells are loaded before the first is
+// used, so that enough loads are in flight to reach the memory's rate; they are combined in the
+// order of the cells (256^3 FP32: one array 45 -> 24 us, three 52 -> 40, 5.0 TB/s).
+template <typename T, typename I, int NA>
 __global__ void __launch_bounds__(RED_TPB) reduce_stage1(RedArgs<T> a)
 {
     __shared__ double sh[RED_TPB / 64];
-    const I n = (I)a.nx * (I)a.ny * (I)a.nz;
-    const I mx = (I)a.mx, sz = (I)a.mx * (I)a.my;
+    constexpr int U = NA == 1 ? 8 : 4;
+    const I n = (I)a.nx * (I)a.ny * (I)a.nz, step = (I)gridDim.x * blockDim.x;
+    I t = (I)blockIdx.x * blockDim.x + threadIdx.x;
+    CellWalk<I> w(t, step, a.nx, a.ny, a.mx, a.my);
     double acc = red_init(a.op);
-    for (I t = (I)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (I)gridDim.x * blockDim.x) {
-        const I c = interior_index<I>(t, (I)a.nx, (I)a.ny, mx, sz);
-        acc = red_combine(a.op, acc, red_map(a.map, a.bufs, (long long)c));
+    while (t < n) {
+        T v[U][NA > 0 ? NA : 1];
+        int cnt = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (t < n) {
+                const I c = w.cell();
+#pragma unroll
+                for (int q = 0; q < NA; ++q)
+                    v[u][q] = a.bufs[q][c];
+                ++cnt;
+            }
+            w.advance();
+            t += step;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < cnt)
+                acc = red_combine(a.op, acc, red_map(a.map, v[u]));
     }
     const double r = block_reduce(a.op, acc, sh);
     if (threadIdx.x == 0)
@@ -314,12 +358,101 @@ void launch_reduce(const T* const* bufs, int map, int op, int nx, int ny, int nz
     int nb = reduce_num_partials(nx, ny, nz);
     if (nb > max_partials)
         nb = max_partials;
-    if (use_index32(nx, ny, nz))
-        hipLaunchKernelGGL((reduce_stage1<T, unsigned>), dim3(nb), dim3(RED_TPB), 0, s, a);
-    else
-        hipLaunchKernelGGL((reduce_stage1<T, unsigned long long>), dim3(nb), dim3(RED_TPB), 0, s, a);
+#define AC_REDUCE(NA)                                                                               \
+    do {                                                                                           \
+        if (use_index32(nx, ny, nz))                                                               \
+            hipLaunchKernelGGL((reduce_stage1<T, unsigned, NA>), dim3(nb), dim3(RED_TPB), 0, s, a); \
+        else                                                                                       \
+            hipLaunchKernelGGL((reduce_stage1<T, unsigned long long, NA>), dim3(nb), dim3(RED_TPB), 0, s, a); \
+    } while (0)
+    switch (red_arrays(map)) {
+    case 1: AC_REDUCE(1); break;
+    case 3: AC_REDUCE(3); break;
+    case 4: AC_REDUCE(4); break;
+    default: AC_REDUCE(0); break;
+    }
+#undef AC_REDUCE
     hipLaunchKernelGGL(reduce_stage2, dim3(1), dim3(RED_TPB), 0, s, (const double*)partials, nb,
                        op, result_dev);
+}
+
+// ---------------------------------------------------------------- marching along z with curl A
+// Kernels that read curl A take 256 columns (numbered x fastest, so no lane is lost to ragged rows) and
+// march them through zchunk planes. The z neighbours of A_x and A_y stay in registers, which leaves 26 of
+// the 36 neighbour loads of a cell. Items (256 columns of one chunk) go to the XCDs in contiguous
+// ranges, workgroup b running on XCD b % 8, so that a row read as a neighbour is in the L2 of the XCD
+// that owns it. Diagnostics 256^3 FP32: 360 us a cell at a time with two divisions for its index and a
+// barrier pair per accumulator at the end; 231 without those and with the ranges; 195 marching (the eight
+// fields read once at 4 TB/s: 134). Reference maxima 128^3 FP32: 376, 32, 28 us.
+struct MarchShape {
+    int zchunk, blocks;
+};
+static MarchShape march_shape(int nx, int ny, int nz)
+{
+    const long long cols = ((long long)nx * ny + RED_TPB - 1) / RED_TPB;
+    // about 1024 items, of at least four planes (six more are loaded to start a chunk)
+    const long long nch = std::max(1ll, std::min(RED_MAX_BLOCKS / cols, (long long)(nz + 3) / 4));
+    const int zc = (int)((nz + nch - 1) / nch);
+    const long long items = cols * ((nz + zc - 1) / zc);
+    return {zc, (int)std::min<long long>(items, reduce_num_partials(nx, ny, nz))};
+}
+
+// Calls f(c, g) for every interior cell c of this workgroup, g[q][ax] = d A_q / d x_ax for q != ax.
+template <typename T, typename I, typename F>
+__device__ __forceinline__ void march_curl(const T* const* A, const Coeffs<T>& C, int nx, int ny, int nz, int mx,
+                                           int my, int zchunk, F&& f)
+{
+    const long long cols = ((long long)nx * ny + RED_TPB - 1) / RED_TPB;
+    const long long items = cols * ((nz + zchunk - 1) / zchunk);
+    long long first = blockIdx.x, last = items, step = gridDim.x;
+    if (gridDim.x % 8 == 0) {
+        const int xcd = blockIdx.x & 7;
+        first = items * xcd / 8 + (blockIdx.x >> 3);
+        last = items * (xcd + 1) / 8;
+        step = gridDim.x >> 3;
+    }
+    const I sy = (I)mx, sz = (I)mx * (I)my;
+    const T* __restrict__ ax = A[0];
+    const T* __restrict__ ay = A[1];
+    const T* __restrict__ az = A[2];
+    auto d1 = [](const T* kk, T p1, T m1, T p2, T m2, T p3, T m3) {
+        return kk[1] * (p1 - m1) + kk[2] * (p2 - m2) + kk[3] * (p3 - m3);
+    };
+    for (long long item = first; item < last; item += step) {
+        const long long col = item % cols * RED_TPB + threadIdx.x;
+        const int z0 = (int)(item / cols) * zchunk;
+        if (col >= (long long)nx * ny)
+            continue;
+        const int z1 = min(z0 + zchunk, nz);
+        I c = (I)((unsigned)col % (unsigned)nx + R) + sy * (I)((unsigned)col / (unsigned)nx + R) + sz * (I)(z0 + R);
+        T qx[7], qy[7];
+#pragma unroll
+        for (int o = 0; o < 6; ++o) {
+            qx[o] = ax[c + o * sz - 3 * sz];
+            qy[o] = ay[c + o * sz - 3 * sz];
+        }
+        for (int k = z0; k < z1; ++k) {
+            qx[6] = ax[c + 3 * sz];
+            qy[6] = ay[c + 3 * sz];
+            T g[3][3];
+            auto along = [&](const T* p, I s, const T* kk) {
+                return d1(kk, p[c + s], p[c - s], p[c + 2 * s], p[c - 2 * s], p[c + 3 * s], p[c - 3 * s]);
+            };
+            g[0][1] = along(ax, sy, C.d1[1]);
+            g[1][0] = along(ay, 1, C.d1[0]);
+            g[2][0] = along(az, 1, C.d1[0]);
+            g[2][1] = along(az, sy, C.d1[1]);
+            g[0][2] = d1(C.d1[2], qx[4], qx[2], qx[5], qx[1], qx[6], qx[0]);
+            g[1][2] = d1(C.d1[2], qy[4], qy[2], qy[5], qy[1], qy[6], qy[0]);
+            f(c, g);
+#pragma unroll
+            for (int o = 0; o < 6; ++o) {
+                qx[o] = qx[o + 1];
+                qy[o] = qy[o + 1];
+            }
+            c += sz;
+        }
+    }
 }
 
 // ---------------------------------------------------------------- diagnostics
@@ -328,7 +461,7 @@ template <typename T>
 struct DiagArgs {
     const T* f[NF];
     Coeffs<T> C;
-    int nx, ny, nz, mx, my;
+    int nx, ny, nz, mx, my, zchunk;
     double* partials;  // DIAG_SLOTS * gridDim.x
 };
 
@@ -345,75 +478,90 @@ __device__ __forceinline__ int diag_op(int slot)
     return r == 0 ? 3 : (r == 1 ? 2 : 1);
 }
 
+// Minima and maxima of the fields are kept in T, which holds them exactly. The 33 accumulators are
+// reduced per wave and exchanged through LDS once.
 template <typename T, typename I>
 __global__ void __launch_bounds__(RED_TPB) diagnostics_stage1(DiagArgs<T> a)
 {
-    __shared__ double sh[RED_TPB / 64];
-    double acc[DIAG_SLOTS];
+    __shared__ double sh[DIAG_SLOTS][RED_TPB / 64];
+    T lo[NF], hi[NF];
+    double sq[NF], acc[DIAG_SLOTS - 3 * NF];
 #pragma unroll
-    for (int q = 0; q < DIAG_SLOTS; ++q)
-        acc[q] = red_init(diag_op(q));
-    const I n = (I)a.nx * (I)a.ny * (I)a.nz;
-    const I sy = (I)a.mx, sz = (I)a.mx * (I)a.my;
-    for (I t = (I)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (I)gridDim.x * blockDim.x) {
-        const I c = interior_index<I>(t, (I)a.nx, (I)a.ny, sy, sz);
+    for (int q = 0; q < NF; ++q) {
+        lo[q] = (T)INFINITY;
+        hi[q] = (T)-INFINITY;
+        sq[q] = 0.0;
+    }
+#pragma unroll
+    for (int q = 3 * NF; q < DIAG_SLOTS; ++q)
+        acc[q - 3 * NF] = red_init(diag_op(q));
+    march_curl<T, I>(a.f + 4, a.C, a.nx, a.ny, a.nz, a.mx, a.my, a.zchunk, [&](I c, const T g[3][3]) {
+        T v[NF];
 #pragma unroll
         for (int q = 0; q < NF; ++q) {
-            const double v = a.f[q][c];
-            acc[q] = fmin(acc[q], v);
-            acc[NF + q] = fmax(acc[NF + q], v);
-            acc[2 * NF + q] += v * v;
+            v[q] = a.f[q][c];
+            lo[q] = fmin(lo[q], v[q]);
+            hi[q] = fmax(hi[q], v[q]);
+            sq[q] += (double)v[q] * (double)v[q];
         }
-        const double ux = a.f[1][c], uy = a.f[2][c], uz = a.f[3][c];
+        const double ux = v[1], uy = v[2], uz = v[3];
         const double u2 = ux * ux + uy * uy + uz * uz;
-        acc[3 * NF + 0] += u2;
-        acc[3 * NF + 1] = fmax(acc[3 * NF + 1], u2);
-        acc[3 * NF + 2] = fmin(acc[3 * NF + 2], u2);
-        const I st[3] = {1, sy, sz};
-        double g[3][3];
-#pragma unroll
-        for (int comp = 0; comp < 3; ++comp) {
-            const T* f = a.f[4 + comp];
-#pragma unroll
-            for (int ax = 0; ax < 3; ++ax) {
-                const I s = st[ax];
-                const T* kk = a.C.d1[ax];
-                g[comp][ax] = (double)(kk[1] * (f[c + s] - f[c - s]) + kk[2] * (f[c + 2 * s] - f[c - 2 * s]) +
-                                       kk[3] * (f[c + 3 * s] - f[c - 3 * s]));
-            }
-        }
-        const double bx = g[2][1] - g[1][2], by = g[0][2] - g[2][0], bz = g[1][0] - g[0][1];
+        acc[0] += u2;
+        acc[1] = fmax(acc[1], u2);
+        acc[2] = fmin(acc[2], u2);
+        const double bx = (double)g[2][1] - (double)g[1][2], by = (double)g[0][2] - (double)g[2][0],
+                     bz = (double)g[1][0] - (double)g[0][1];
         const double b2 = bx * bx + by * by + bz * bz;
-        acc[3 * NF + 3] += b2;
-        acc[3 * NF + 4] = fmax(acc[3 * NF + 4], b2);
-        acc[3 * NF + 5] = fmin(acc[3 * NF + 5], b2);
+        acc[3] += b2;
+        acc[4] = fmax(acc[4], b2);
+        acc[5] = fmin(acc[5], b2);
         // Alfven speed |B| / sqrt(rho), rho = exp(lnrho) (ref acc-runtime/stdlib/map.h:121-134)
-        const double va2 = b2 / exp((double)a.f[0][c]);
-        acc[3 * NF + 6] += va2;
-        acc[3 * NF + 7] = fmax(acc[3 * NF + 7], va2);
-        acc[3 * NF + 8] = fmin(acc[3 * NF + 8], va2);
-    }
+        const double va2 = b2 / exp((double)v[0]);
+        acc[6] += va2;
+        acc[7] = fmax(acc[7], va2);
+        acc[8] = fmin(acc[8], va2);
+    });
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
     for (int q = 0; q < DIAG_SLOTS; ++q) {
-        const double r = block_reduce(diag_op(q), acc[q], sh);
-        if (threadIdx.x == 0)
-            a.partials[(long long)q * gridDim.x + blockIdx.x] = r;
-        __syncthreads();
+        double r;
+        if (q < 2 * NF) {
+            T m = q < NF ? lo[q % NF] : hi[q % NF];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+                m = q < NF ? fmin(m, __shfl_xor(m, off, 64)) : fmax(m, __shfl_xor(m, off, 64));
+            r = m;
+        }
+        else {
+            r = q < 3 * NF ? sq[q % NF] : acc[q < 3 * NF ? 0 : q - 3 * NF];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+                r = red_combine(diag_op(q), r, __shfl_xor(r, off, 64));
+        }
+        if (lane == 0)
+            sh[q][wid] = r;
+    }
+    __syncthreads();
+    const int q = threadIdx.x;
+    if (q < DIAG_SLOTS) {
+        double r = red_init(diag_op(q));
+        for (int k = 0; k < RED_TPB / 64; ++k)
+            r = red_combine(diag_op(q), r, sh[q][k]);
+        a.partials[(long long)q * gridDim.x + blockIdx.x] = r;
     }
 }
 
+// One workgroup per slot (one for all slots in turn took 79 us at 256^3, this 4).
 __global__ void __launch_bounds__(RED_TPB) diagnostics_stage2(const double* partials, int np, double* out)
 {
     __shared__ double sh[RED_TPB / 64];
-    for (int q = 0; q < DIAG_SLOTS; ++q) {
-        const int op = diag_op(q);
-        double acc = red_init(op);
-        for (int t = threadIdx.x; t < np; t += blockDim.x)
-            acc = red_combine(op, acc, partials[(long long)q * np + t]);
-        const double r = block_reduce(op, acc, sh);
-        if (threadIdx.x == 0)
-            out[q] = r;
-        __syncthreads();
-    }
+    const int q = blockIdx.x, op = diag_op(q);
+    double acc = red_init(op);
+    for (int t = threadIdx.x; t < np; t += blockDim.x)
+        acc = red_combine(op, acc, partials[(long long)q * np + t]);
+    const double r = block_reduce(op, acc, sh);
+    if (threadIdx.x == 0)
+        out[q] = r;
 }
 
 template <typename T>
@@ -430,19 +578,30 @@ void launch_diagnostics(const T* const* fields, const Coeffs<T>& C, int nx, int 
     a.mx = nx + 2 * R;
     a.my = ny + 2 * R;
     a.partials = partials;
-    int nb = reduce_num_partials(nx, ny, nz);
-    if (nb * DIAG_SLOTS > max_partials)
-        nb = max_partials / DIAG_SLOTS;
+    const MarchShape shape = march_shape(nx, ny, nz);
+    a.zchunk = shape.zchunk;
+    const int nb = std::min(shape.blocks, max_partials / DIAG_SLOTS);
     if (use_index32(nx, ny, nz))
         hipLaunchKernelGGL((diagnostics_stage1<T, unsigned>), dim3(nb), dim3(RED_TPB), 0, s, a);
     else
         hipLaunchKernelGGL((diagnostics_stage1<T, unsigned long long>), dim3(nb), dim3(RED_TPB), 0,
                            s, a);
-    hipLaunchKernelGGL(diagnostics_stage2, dim3(1), dim3(RED_TPB), 0, s, (const double*)partials,
+    hipLaunchKernelGGL(diagnostics_stage2, dim3(DIAG_SLOTS), dim3(RED_TPB), 0, s, (const double*)partials,
                        nb, out_dev);
 }
 
 // ---------------------------------------------------------------- max |u|^2
+// Block-level max of a non-negative double, one atomic per workgroup at most (two per wave were most of
+// the 376 us that the reference timestep's maxima took at 128^3).
+__device__ __forceinline__ void block_max_to_global(double v, unsigned long long* dst)
+{
+    __shared__ double sh[RED_TPB / 64];
+    __syncthreads();
+    const double r = block_reduce(2, v, sh);
+    if (threadIdx.x == 0)
+        atomic_max_nonneg(dst, r);
+}
+
 template <typename T>
 struct UmaxArgs {
     const T* u[3];
@@ -453,15 +612,15 @@ struct UmaxArgs {
 template <typename T, typename I>
 __global__ void __launch_bounds__(RED_TPB) umax2_kernel(UmaxArgs<T> a)
 {
-    const I n = (I)a.nx * (I)a.ny * (I)a.nz;
-    const I mx = (I)a.mx, sz = (I)a.mx * (I)a.my;
+    const I n = (I)a.nx * (I)a.ny * (I)a.nz, step = (I)gridDim.x * blockDim.x;
+    I t = (I)blockIdx.x * blockDim.x + threadIdx.x;
     double m = 0.0;
-    for (I t = (I)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (I)gridDim.x * blockDim.x) {
-        const I c = interior_index<I>(t, (I)a.nx, (I)a.ny, mx, sz);
+    for (CellWalk<I> w(t, step, a.nx, a.ny, a.mx, a.my); t < n; t += step, w.advance()) {
+        const I c = w.cell();
         const double x = a.u[0][c], y = a.u[1][c], z = a.u[2][c];
         m = fmax(m, x * x + y * y + z * z);
     }
-    wave_max_to_global(m, a.umax2);
+    block_max_to_global(m, a.umax2);
 }
 
 template <typename T>
@@ -491,7 +650,7 @@ template <typename T>
 struct CflArgs {
     const T* f[NF];
     Coeffs<T> C;
-    int nx, ny, nz, mx, my;
+    int nx, ny, nz, mx, my, zchunk;
     int mode;
     double cs2;
     unsigned long long* out;  // pair
@@ -500,34 +659,25 @@ struct CflArgs {
 template <typename T, typename I>
 __global__ void __launch_bounds__(RED_TPB) cfl_state_kernel(CflArgs<T> a)
 {
-    const I n = (I)a.nx * (I)a.ny * (I)a.nz;
-    const I sy = (I)a.mx, sz = (I)a.mx * (I)a.my;
     double mx_ = 0.0, my_ = 0.0;
-    for (I t = (I)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (I)gridDim.x * blockDim.x) {
-        const I c = interior_index<I>(t, (I)a.nx, (I)a.ny, sy, sz);
-        const I st[3] = {1, sy, sz};
+    march_curl<T, I>(a.f + 4, a.C, a.nx, a.ny, a.nz, a.mx, a.my, a.zchunk, [&](I c, const T g[3][3]) {
         CellDerivs<T> d;
         d.lr = a.f[0][c];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             d.u[q] = a.f[1 + q][c];
-            const T* f = a.f[4 + q];
 #pragma unroll
-            for (int ax = 0; ax < 3; ++ax) {
-                const I s = st[ax];
-                const T* kk = a.C.d1[ax];
-                d.ga[q][ax] = kk[1] * (f[c + s] - f[c - s]) + kk[2] * (f[c + 2 * s] - f[c - 2 * s]) +
-                              kk[3] * (f[c + 3 * s] - f[c - 3 * s]);
-            }
+            for (int ax = 0; ax < 3; ++ax)
+                d.ga[q][ax] = ax == q ? T(0) : g[q][ax];
         }
         double x, y;
         cfl_cell<T>(a.mode, a.cs2, d, x, y);
         mx_ = fmax(mx_, x);
         my_ = fmax(my_, y);
-    }
-    wave_max_to_global(mx_, a.out);
+    });
+    block_max_to_global(mx_, a.out);
     if (a.mode == 1)
-        wave_max_to_global(my_, a.out + 1);
+        block_max_to_global(my_, a.out + 1);
 }
 
 template <typename T>
@@ -546,8 +696,9 @@ void launch_cfl_state(const T* const* fields, const Coeffs<T>& C, int nx, int ny
     a.mode = mode;
     a.cs2 = cs2;
     a.out = out;
-    const long long n = (long long)nx * ny * nz;
-    const int nb = (int)std::min<long long>((n + RED_TPB - 1) / RED_TPB, 4096);
+    const MarchShape shape = march_shape(nx, ny, nz);
+    a.zchunk = shape.zchunk;
+    const int nb = shape.blocks;
     if (use_index32(nx, ny, nz))
         hipLaunchKernelGGL((cfl_state_kernel<T, unsigned>), dim3(nb), dim3(RED_TPB), 0, s, a);
     else
@@ -588,51 +739,56 @@ void launch_zero_comp_field(void* slab, size_t count, int kahan_bits, int q, hip
 // ref mhdsolver.ac:286-331 (helical_forcing, forcing) and :614-631 (added to u after the final
 // update of substep 2). The geometry and the mode are evaluated in FP64, the force is rounded to
 // AcReal and added to the stored u in AcReal, as the reference adds forcing_step to rk3_final.
+// A workgroup marches its 64 x 4 columns through zchunk planes, so the phase and the x and y parts of
+// k . y, with their FP64 divisions and sines, are taken once per column, and max |u|^2 makes one atomic
+// per workgroup (128^3 FP32: 23 -> 18 us; u alone, read and written, is 50 MB).
 template <typename T>
-__global__ void __launch_bounds__(256) forcing_kernel(ForcingArgs<T> a)
+__global__ void __launch_bounds__(RED_TPB) forcing_kernel(ForcingArgs<T> a, int zchunk)
 {
-    const int i = threadIdx.x + blockIdx.x * blockDim.x;
-    const int j = threadIdx.y + blockIdx.y * blockDim.y;
-    const int k = blockIdx.z;
-    const bool inside = i < a.nx && j < a.ny && k < a.nz;
+    const int i = (int)(threadIdx.x & 63) + blockIdx.x * 64;
+    const int j = (int)(threadIdx.x >> 6) + blockIdx.y * (RED_TPB / 64);
+    const int k0 = blockIdx.z * zchunk;
+    const int k1 = i < a.nx && j < a.ny ? min(k0 + zchunk, a.nz) : k0;
     const double dt = (double)solve_dt(a.s);
     const double t0 = a.time_acc ? a.t_base + (*a.time_acc - dt) : a.t_base;
+    const bool on = t0 > a.switch_time;
     double u2 = 0.0;
-    if (inside) {
+    // y = 2 pi xx / (ds ngrid), xx = (global index - nmin) ds
+    auto part = [&](int d, int g, int ng) {
+        return a.k[d] * (2.0 * M_PI * (((double)g * a.ds[d]) / (a.ds[d] * (double)ng)));
+    };
+    const double kxy = (0.0 + part(0, a.gx0 + i, a.ngx)) + part(1, a.gy0 + j, a.ngy);
+    double sp, cp;
+    sincos(a.phase, &sp, &cp);
+    const double amp = sqrt(dt) * a.nn;
+    for (int k = k0; k < k1; ++k) {
         const long long c = (long long)(i + R) + (long long)a.mx * (j + R) + a.sz * (k + R);
         T u[3] = {a.uu[0][c], a.uu[1][c], a.uu[2][c]};
-        if (t0 > a.switch_time) {
-            // y = 2 pi xx / (ds ngrid), xx = (global index - nmin) ds
-            const double g[3] = {(double)(a.gx0 + i), (double)(a.gy0 + j), (double)(a.gz0 + k)};
-            const int ng[3] = {a.ngx, a.ngy, a.ngz};
-            double kdy = 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                kdy += a.k[d] * (2.0 * M_PI * ((g[d] * a.ds[d]) / (a.ds[d] * (double)ng[d])));
-            double sk, ck, sp, cp;
-            sincos(kdy, &sk, &ck);
-            sincos(a.phase, &sp, &cp);
+        if (on) {
+            double sk, ck;
+            sincos(kxy + part(2, a.gz0 + k, a.ngz), &sk, &ck);
             const double re = ck * cp - sk * sp;
             const double im = ck * sp + sk * cp;
-            const double amp = sqrt(dt) * a.nn;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 u[d] = u[d] + (T)(amp * (a.fre[d] * re - a.fim[d] * im));
                 a.uu[d][c] = u[d];
             }
         }
-        u2 = (double)u[0] * (double)u[0] + (double)u[1] * (double)u[1] + (double)u[2] * (double)u[2];
+        u2 = fmax(u2, (double)u[0] * (double)u[0] + (double)u[1] * (double)u[1] + (double)u[2] * (double)u[2]);
     }
     if (a.umax2_next != nullptr)
-        wave_max_to_global(u2, a.umax2_next);
+        block_max_to_global(u2, a.umax2_next);
 }
 
 template <typename T>
 void launch_forcing(const ForcingArgs<T>& a, hipStream_t s)
 {
-    const dim3 tpb(64, 4, 1);
-    const dim3 bpg((unsigned)((a.nx + 63) / 64), (unsigned)((a.ny + 3) / 4), (unsigned)a.nz);
-    hipLaunchKernelGGL((forcing_kernel<T>), bpg, tpb, 0, s, a);
+    // planes per workgroup: up to 8 where that leaves four workgroups for each CU
+    const long long columns = (long long)((a.nx + 63) / 64) * ((a.ny + 3) / 4);
+    const int zc = (int)std::max(1ll, std::min(8ll, columns * a.nz / 1024));
+    const dim3 bpg((unsigned)((a.nx + 63) / 64), (unsigned)((a.ny + 3) / 4), (unsigned)((a.nz + zc - 1) / zc));
+    hipLaunchKernelGGL((forcing_kernel<T>), bpg, dim3(RED_TPB), 0, s, a, zc);
 }
 
 template void launch_forcing<AcRealT>(const ForcingArgs<AcRealT>&, hipStream_t);

@@ -67,7 +67,6 @@ struct device_s {
     // reductions and device-resident scalars
     double* partials;
     int max_partials;
-    double* dres;                 // [0] reduce result, [1..] diagnostics
     unsigned long long* umax2;    // two slot pairs (x, y) of the timestep reductions
     double* time_acc;
     int cfl_cur;
@@ -75,7 +74,7 @@ struct device_s {
     int cfl_mode;                 // 0 courant, 1 reference (2 when AC_additive_timestep)
     bool periodic_fused;          // substeps read the periodic images (no halo fill before them)
     bool forcing_time_acc;        // forcing start time = AC_current_time + time_acc - dt
-    double* host_pinned;          // staging for small D2H reads
+    double* host_pinned;          // results of reductions, staging for small D2H reads
     // stencil coefficients (grid spacing folded in), set by acDeviceLoadStencilsFromConfig
     Coeffs<AcReal> C;
     // launch shape
@@ -408,7 +407,6 @@ AcResult acDeviceCreate(const int id, const AcMeshInfo device_config, Device* de
     const int3 n = d->local_config.int3_params[AC_nlocal];
     d->max_partials = std::max(reduce_num_partials(n.x, n.y, n.z), 1) * kDiagSlots;
     AC_HIP_CHECK(hipMalloc(&d->partials, sizeof(double) * d->max_partials));
-    AC_HIP_CHECK(hipMalloc(&d->dres, sizeof(double) * (1 + kDiagSlots)));
     AC_HIP_CHECK(hipMalloc(&d->umax2, sizeof(unsigned long long) * 4));
     AC_HIP_CHECK(hipMalloc(&d->time_acc, sizeof(double)));
     launch_zero_bytes(d->umax2, sizeof(unsigned long long) * 4, s0);
@@ -440,7 +438,6 @@ AcResult acDeviceDestroy(Device* device_ptr)
     if (d->slab_comp)
         hipFree(d->slab_comp);
     hipFree(d->partials);
-    hipFree(d->dres);
     hipFree(d->umax2);
     hipFree(d->time_acc);
     hipHostFree(d->host_pinned);
@@ -922,11 +919,10 @@ AcResult acDevicePeriodicBoundconds(const Device d, const Stream stream, const V
     return periodic_fill(d, stream, d->in, NF, start, end, "acDevicePeriodicBoundconds");
 }
 
-// The two-stage reduction with its partial results in `partials` (max_partials of them) and the
-// final value in *result_dev, both device memory.
-static AcResult reduce_into(Device d, const Stream stream, const AcReduction r, int map,
-                            const VertexBufferHandle* h, int nh, bool post, double* partials,
-                            int max_partials, double* result_dev, AcReal* result)
+// The two-stage reduction. Its second stage writes the result straight into pinned host memory (a copy
+// after it was a launch of its own, 10 us at every size).
+static AcResult reduce_common(Device d, const Stream stream, const AcReduction r, int map,
+                              const VertexBufferHandle* h, int nh, bool post, AcReal* result)
 {
     for (int q = 0; q < nh; ++q)
         if ((int)h[q] < 0 || (int)h[q] >= NF)
@@ -939,22 +935,15 @@ static AcResult reduce_into(Device d, const Stream stream, const AcReduction r, 
     for (int q = 0; q < nh; ++q)
         bufs[q] = d->in[h[q]];
     const int3 n = d->local_config.int3_params[AC_nlocal];
-    launch_reduce<AcReal>(bufs, (int)map, (int)r.reduce_op, n.x, n.y, n.z, partials, max_partials,
-                          result_dev, s);
+    launch_reduce<AcReal>(bufs, (int)map, (int)r.reduce_op, n.x, n.y, n.z, d->partials,
+                          d->max_partials, d->host_pinned, s);
     AC_HIP_CHECK(hipGetLastError());
-    AC_HIP_CHECK(hipMemcpyAsync(d->host_pinned, result_dev, sizeof(double), hipMemcpyDeviceToHost, s));
     AC_HIP_CHECK(hipStreamSynchronize(s));
     double v = d->host_pinned[0];
     if (post && r.post_processing_op == AC_RMS)
         v = sqrt(v / ((double)n.x * n.y * n.z));
     *result = (AcReal)v;
     return AC_SUCCESS;
-}
-
-static AcResult reduce_common(Device d, const Stream stream, const AcReduction r, int map,
-                              const VertexBufferHandle* h, int nh, bool post, AcReal* result)
-{
-    return reduce_into(d, stream, r, map, h, nh, post, d->partials, d->max_partials, d->dres, result);
 }
 
 AcResult acDeviceReduceScalNoPostProcessing(const Device d, const Stream stream,
@@ -1178,10 +1167,8 @@ AcResult acDeviceReduceDiagnostics(const Device d, const Stream stream, AcDiagno
     const AcReal* f[NF];
     for (int q = 0; q < NF; ++q)
         f[q] = d->in[q];
-    launch_diagnostics<AcReal>(f, d->C, n.x, n.y, n.z, d->partials, d->max_partials, d->dres + 1, s);
+    launch_diagnostics<AcReal>(f, d->C, n.x, n.y, n.z, d->partials, d->max_partials, d->host_pinned, s);
     AC_HIP_CHECK(hipGetLastError());
-    AC_HIP_CHECK(hipMemcpyAsync(d->host_pinned, d->dres + 1, sizeof(double) * kDiagSlots,
-                                hipMemcpyDeviceToHost, s));
     AC_HIP_CHECK(hipStreamSynchronize(s));
     const double* v = d->host_pinned;
     const double inv_n = 1.0 / ((double)n.x * n.y * n.z);

@@ -478,10 +478,13 @@ __device__ __forceinline__ T solve_dt(const SolveArgs<T>& a)
                      a.cfl_cs2, a.cfl_cdtv, a.cfl_visc);
 }
 
-// Block-wide max of |u|^2 into umax2_next (step 2 of the device-dt path), plus time.
+// Max of a non-negative double into *addr (double bits). Atomics on one address from eight XCDs meet in
+// memory one by one, so a value that is no larger than what a load finds there makes none.
 __device__ __forceinline__ void atomic_max_nonneg(unsigned long long* addr, double v)
 {
-    atomicMax(addr, (unsigned long long)__double_as_longlong(v));
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    if (bits > __hip_atomic_load(addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(addr, bits);
 }
 
 }  // namespace acamd
