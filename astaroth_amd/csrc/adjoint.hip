@@ -26,7 +26,8 @@ struct AdjArgs {
     SolveArgs<T> s;        // f = s.in (halos filled), coefficients, parameters, alpha, beta
     T* lf;                 // adjoint of f, NF slabs of m^3, updated in place
     T* lw;                 // adjoint of w, updated in place
-    T* g;                  // NG slabs of m^3 (derivative adjoints)
+    T* g;                  // derivative adjoints, NG fields
+    long long g_row, g_plane, g_field;  // strides of g (values)
     double* partials;      // 2 per block (nu, eta)
     const T* df_in;        // tangent: df (halos filled)
     T* df_out;             // tangent: df'
@@ -157,42 +158,101 @@ __global__ void __launch_bounds__(256) tangent_kernel(AdjArgs<T> A)
     }
 }
 
-// ---------------------------------------------------------------- adjoint (A): local part
-template <typename T, bool UPWD, bool ENTROPY>
-__global__ void __launch_bounds__(256) adjoint_local_kernel(AdjArgs<T> A)
+// This wave's memory operations and LDS reads are done, then the workgroup barrier.
+__device__ __forceinline__ void memory_barrier()
 {
-    __shared__ double sh[2][4];
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// ---------------------------------------------------------------- adjoint (A): local part
+// One cell per thread on blocks of 16 x 4 x 4 cells, in FP64 and for FP32 grids that the tiled form's 64 x 4
+// columns do not divide. The block's box of the state, with its radius-3 halo, is DMA'd into LDS and all
+// stencils read it there (22 x 10 x 10 cells of 8 fields: 69 loads per cell, from L2 mostly, in place of
+// the 230 that the stencils make). 16 columns are one 64-byte line of the derivative adjoints in FP32.
+// Reading the stencils from global memory it took 163 us at 72 x 60 x 50 FP64, now 70; whole adjoint
+// substep 144 x 128 x 112 FP32 1206 -> 574 us. Two workgroups share a CU in FP32 (222 VGPRs), one in FP64;
+// their load, stencil and store phases overlap only with each other's.
+constexpr int BX = 16, BY = 4, BZ = 4;
+constexpr int BLX = BX + 2 * R, BLY = BY + 2 * R, BLZ = BZ + 2 * R;
+
+static long long adjoint_local_blocks(int nx, int ny, int nz)
+{
+    return (long long)((nx + BX - 1) / BX) * ((ny + BY - 1) / BY) * ((nz + BZ - 1) / BZ);
+}
+
+template <typename T, bool UPWD, bool ENTROPY>
+__global__ void __launch_bounds__(BX * BY * BZ) adjoint_local_kernel(AdjArgs<T> A)
+{
+    constexpr int NW = BX * BY * BZ / 64;
+    constexpr int WPE = (int)sizeof(T) / 4;
+    constexpr int BOX = BLX * BLY * BLZ * WPE;                    // dwords of a field's box
+    constexpr int NR = ((BOX + 63) / 64 + NW - 1) / NW;           // DMA rounds per wave
+    constexpr int LPS = NR * NW * 64 / WPE;                       // padded field stride in LDS (values)
+    __shared__ T lds[NF * LPS];
+    __shared__ double sh[2][NW];
     const SolveArgs<T>& a = A.s;
-    bool active;
-    long long c;
-    cell_index(a, active, c);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // each XCD takes a contiguous range of blocks, whose neighbours then share its L2
+    const int nb = (int)gridDim.x;
+    const int bid = (nb & 7) == 0 ? ((int)blockIdx.x & 7) * (nb >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    const int nbx = (a.nx + BX - 1) / BX, nby = (a.ny + BY - 1) / BY;
+    const int x0 = bid % nbx * BX, y0 = bid / nbx % nby * BY, z0 = bid / (nbx * nby) * BZ;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        int d = (wave + r * NW) * 64 + lane;
+        if (d >= BOX)
+            d = 0;  // padding lanes re-read dword 0 of the box
+        const int e = d / WPE, wd = d - e * WPE;
+        const int lz = e / (BLX * BLY), ly = e / BLX % BLY, lx = e % BLX;
+        // past the array (blocks at the upper edges): the last cell, unused
+        const long long src = min(x0 + lx, a.mx - 1) + (long long)a.mx * min(y0 + ly, a.my - 1) +
+                              a.sz * min(z0 + lz, a.mz - 1);
+#pragma unroll
+        for (int q = 0; q < NF; ++q)
+            __builtin_amdgcn_global_load_lds((const void*)((const char*)(a.in[q] + src) + 4 * wd),
+                                             (lds_ptr_t)(lds + q * LPS + (wave + r * NW) * (64 / WPE)), 4, 0, 0);
+    }
+    const int tx = tid % BX, ty = tid / BX % BY, tz = tid / (BX * BY);
+    const int i = x0 + tx, j = y0 + ty, k = z0 + tz;
+    const bool active = i < a.nx && j < a.ny && k < a.nz;
+    const long long c = active ? (long long)(i + R) + (long long)a.mx * (j + R) + a.sz * (k + R) : 0;
+    T lf[NF], mu[NF];
+    if (active) {
+#pragma unroll
+        for (int q = 0; q < NF; ++q) {
+            const long long o = (long long)q * A.count + c;
+            lf[q] = A.lf[o];
+            mu[q] = A.lw[o] + a.beta * lf[q];
+        }
+    }
+    memory_barrier();
     double pnu = 0.0, peta = 0.0;
     if (active) {
         CellDerivs<T> d, ad;
         UpwindDirs<T> up, aup;
-        gather<T, UPWD>(a.in, c, a.mx, a.sz, a.C, d, up);
-        T mu[NF];
+        const T* f[NF];
 #pragma unroll
-        for (int q = 0; q < NF; ++q) {
-            const long long o = (long long)q * A.count + c;
-            mu[q] = A.lw[o] + a.beta * A.lf[o];
-        }
+        for (int q = 0; q < NF; ++q)
+            f[q] = lds + q * LPS;
+        gather<T, UPWD>(f, (tx + R) + BLX * (ty + R) + BLX * BLY * (tz + R), BLX, BLX * BLY, a.C, d, up);
         if (!ENTROPY)
             mu[7] = T(0);
         T anu, aeta;
         mhd_rhs_vjp<T, UPWD, ENTROPY>(d, up, mu, a.P, ad, aup, anu, aeta);
         pnu = (double)a.dt * (double)anu;
         peta = (double)a.dt * (double)aeta;
-        T* g = A.g;
-        const long long n = A.count;
-        put_derivative_adjoints<UPWD>(ad, aup, [&](int k, T v) { g[(long long)k * n + c] = v; });
+        T* g = A.g + i + A.g_row * j + A.g_plane * k;
+        put_derivative_adjoints<UPWD>(ad, aup, [&](int f, T v) { g[f * A.g_field] = v; });
 #pragma unroll
         for (int q = 0; q < NF; ++q) {
-            const long long o = (long long)q * n + c;
-            const T lfo = A.lf[o];
+            const long long o = (long long)q * A.count + c;
             A.lw[o] = a.alpha * mu[q];
             if (q < 4 || (q == 7 && ENTROPY))
-                A.lf[o] = lfo + a.dt * value_adjoint(ad, q);
+                A.lf[o] = lf[q] + a.dt * value_adjoint(ad, q);
         }
     }
     // block sums of the parameter sensitivities (FP64)
@@ -201,22 +261,19 @@ __global__ void __launch_bounds__(256) adjoint_local_kernel(AdjArgs<T> A)
         pnu += __shfl_xor(pnu, off, 64);
         peta += __shfl_xor(peta, off, 64);
     }
-    const int tid = threadIdx.x + blockDim.x * threadIdx.y;
-    if ((tid & 63) == 0) {
-        sh[0][tid >> 6] = pnu;
-        sh[1][tid >> 6] = peta;
+    if (lane == 0) {
+        sh[0][wave] = pnu;
+        sh[1][wave] = peta;
     }
     __syncthreads();
     if (tid == 0) {
-        const int nw = (blockDim.x * blockDim.y + 63) >> 6;
         double s0 = 0.0, s1 = 0.0;
-        for (int w = 0; w < nw; ++w) {
+        for (int w = 0; w < NW; ++w) {
             s0 += sh[0][w];
             s1 += sh[1][w];
         }
-        const long long b = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
-        A.partials[2 * b + 0] = s0;
-        A.partials[2 * b + 1] = s1;
+        A.partials[2 * (long long)blockIdx.x + 0] = s0;
+        A.partials[2 * (long long)blockIdx.x + 1] = s1;
     }
 }
 
@@ -376,15 +433,6 @@ struct TransposeTile {
 };
 constexpr int most_staged(bool upwd) { return upwd ? 8 : 6; }
 
-// This wave's memory operations and LDS reads are done, then the workgroup barrier.
-__device__ __forceinline__ void transpose_barrier()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 __device__ __forceinline__ int wrap_index(int i, int n)
 {
     while (i < 0)
@@ -426,11 +474,11 @@ __device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T*
         const int e = d / WPE, wd = d - e * WPE;
         const int ly = e / LX, lx = e - ly * LX;
         const int gx = wrap_index(x0 + lx - R, a.nx), gy = wrap_index(y0 + ly - R, a.ny);
-        g_off[r] = (unsigned)(((gx + R) + sy * (gy + R)) * (int)sizeof(T) + 4 * wd);
+        g_off[r] = (unsigned)((gx + (int)A.g_row * gy) * (int)sizeof(T) + 4 * wd);
     }
-    // byte offset of interior plane p (z wrapped periodically) within a field
+    // byte offset of interior plane p (z wrapped periodically) within a field of g
     auto plane_b = [&](int p) {
-        return sz * (long long)(wrap_index(p, a.nz) + R) * (long long)sizeof(T);
+        return A.g_plane * (long long)wrap_index(p, a.nz) * (long long)sizeof(T);
     };
     auto dma_plane = [&](int p, T* dst, long long nb) {
         const char* pb = (const char*)A.g + plane_b(p);
@@ -448,8 +496,9 @@ __device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T*
 
     const int ctr = (ty + R) * LX + (tx + R);
     // columns past the grid read a column inside it and write nothing
-    const unsigned colb0 = (unsigned)((((inside ? x0 + tx : 0) + R) + sy * ((inside ? y0 + ty : 0) + R)) *
-                                      (int)sizeof(T));
+    const int cx = inside ? x0 + tx : 0, cy = inside ? y0 + ty : 0;
+    const unsigned colb0 = (unsigned)(((cx + R) + sy * (cy + R)) * (int)sizeof(T));
+    const unsigned colg0 = (unsigned)((cx + (int)A.g_row * cy) * (int)sizeof(T));
     T acc[7];
 #pragma unroll
     for (int k = 0; k < 7; ++k)
@@ -471,19 +520,20 @@ __device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T*
     };
 
     {
-        const long long nb = A.count * (long long)sizeof(T);
-        dma_plane(z0 - R, lds0, nb);
-        load_cols(z0 - R, nb, colb0, col);
+        const long long gb = A.g_field * (long long)sizeof(T);
+        dma_plane(z0 - R, lds0, gb);
+        load_cols(z0 - R, gb, colg0, col);
     }
-    transpose_barrier();
+    memory_barrier();
     const int np = z1 - z0 + 2 * R;
     auto step = [&](int it, const T* lds, T* next) {
         const int p = z0 - R + it;
         const long long nb = opaque_s64(A.count * (long long)sizeof(T));
+        const long long gb = opaque_s64(A.g_field * (long long)sizeof(T));
         const unsigned colb = opaque(colb0);
         if (it + 1 < np) {
-            dma_plane(p + 1, next, nb);
-            load_cols(p + 1, nb, colb, coln);
+            dma_plane(p + 1, next, gb);
+            load_cols(p + 1, gb, opaque(colg0), coln);
             if (it + 1 >= 2 * R)
                 lfn = *(const T*)((const char*)A.lf + out_off(it + 1, nb, colb));
         }
@@ -593,7 +643,7 @@ __device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T*
             col[c] = coln[c];
         lfc = lfn;
         // plane p + 1 has landed and every wave is done with this one
-        transpose_barrier();
+        memory_barrier();
     };
     for (int it = 0; it < np; it += 2) {
         step(it, lds0, lds1);
@@ -659,9 +709,10 @@ void launch_tangent(const AdjArgs<T>& A, bool upwd, bool entropy, hipStream_t s)
     else hipLaunchKernelGGL((tangent_kernel<T, false, false>), bpg, tpb, 0, s, A);
 }
 
+// At least the workgroups of stage (A) in either form.
 long long adjoint_num_blocks(int nx, int ny, int nz)
 {
-    return (long long)((nx + 63) / 64) * ((ny + 3) / 4) * nz;
+    return std::max((long long)((nx + 63) / 64) * ((ny + 3) / 4) * nz, adjoint_local_blocks(nx, ny, nz));
 }
 
 struct TransposeShape {
@@ -702,21 +753,16 @@ template <typename T>
 void launch_adjoint(const AdjArgs<T>& A, bool upwd, bool entropy, double* param_grad,
                     hipStream_t s)
 {
-    const dim3 tpb(64, 4, 1), bpg = grid_of(A.s);
-#define AC_ADJ(K)                                                                                  \
-    do {                                                                                           \
-        if (upwd && entropy) hipLaunchKernelGGL((K<T, true, true>), bpg, tpb, 0, s, A);            \
-        else if (upwd) hipLaunchKernelGGL((K<T, true, false>), bpg, tpb, 0, s, A);                 \
-        else if (entropy) hipLaunchKernelGGL((K<T, false, true>), bpg, tpb, 0, s, A);              \
-        else hipLaunchKernelGGL((K<T, false, false>), bpg, tpb, 0, s, A);                          \
-    } while (0)
-    // (A) derivative adjoints: the tiled kernel where the grid fits its 64 x 4 tiles (it has at
-    // most as many blocks, so its partial sums fit the same workspace), else one cell per thread
+    // (A) derivative adjoints: the tiled kernel where the grid fits its 64 x 4 tiles, else blocks
     long long nb = 0;
-    const AdjLocal<T> xl{A.g, A.lf, A.lw, A.partials};
+    const AdjLocal<T> xl{A.g, A.g_row, A.g_plane, A.g_field, A.lf, A.lw, A.partials};
     if (!launch_adjoint_local_tiled<T>(A.s, xl, upwd, entropy, s, &nb)) {
-        AC_ADJ(adjoint_local_kernel);
-        nb = (long long)bpg.x * bpg.y * bpg.z;
+        nb = adjoint_local_blocks(A.s.nx, A.s.ny, A.s.nz);
+        const dim3 bpg((unsigned)nb), tpb(BX * BY * BZ);
+        if (upwd && entropy) hipLaunchKernelGGL((adjoint_local_kernel<T, true, true>), bpg, tpb, 0, s, A);
+        else if (upwd) hipLaunchKernelGGL((adjoint_local_kernel<T, true, false>), bpg, tpb, 0, s, A);
+        else if (entropy) hipLaunchKernelGGL((adjoint_local_kernel<T, false, true>), bpg, tpb, 0, s, A);
+        else hipLaunchKernelGGL((adjoint_local_kernel<T, false, false>), bpg, tpb, 0, s, A);
     }
     double* ranges = A.partials + 2 * nb;
     hipLaunchKernelGGL(adjoint_param_stage1, dim3(PARAM_RANGES), dim3(256), 0, s,
@@ -744,7 +790,6 @@ void launch_adjoint(const AdjArgs<T>& A, bool upwd, bool entropy, double* param_
         AC_TRANSPOSE(64);
 #endif
 #undef AC_TRANSPOSE
-#undef AC_ADJ
 }
 
 int adjoint_num_fields() { return NG; }
@@ -766,13 +811,24 @@ int device_id(Device d);
 
 using namespace acamd;
 
+// Layout of the derivative adjoints in the workspace: no halo, rows on 64-byte lines, so that stage (A)'s
+// 47 stores per cell write whole lines (rows at the state's odd pitch share lines with their neighbours).
+// Whole adjoint substep FP32: 256^3 2931 -> 2779 us, 128^3 421 -> 403. An odd number of lines per row
+// (256^3 3014 us) and a skew between the fields (2827) were slower.
+struct AdjLayout {
+    long long row, plane, field;  // strides in values
+};
+static AdjLayout adjoint_layout(const int3 n)
+{
+    const long long line = 64 / (long long)sizeof(AcReal);
+    const long long row = (n.x + line - 1) / line * line;
+    return {row, row * n.y, row * n.y * n.z};
+}
+
 extern "C" size_t acAdjointWorkspaceBytes(const Device d)
 {
-    const AcMeshInfo info = acDeviceGetLocalConfig(d);
-    const int3 m = info.int3_params[AC_mlocal];
-    const int3 n = info.int3_params[AC_nlocal];
-    const size_t count = (size_t)m.x * m.y * m.z;
-    const size_t g = count * NG * sizeof(AcReal);
+    const int3 n = acDeviceGetLocalConfig(d).int3_params[AC_nlocal];
+    const size_t g = (size_t)adjoint_layout(n).field * NG * sizeof(AcReal);
     const size_t partials =
         ((size_t)adjoint_num_blocks(n.x, n.y, n.z) + PARAM_RANGES) * 2 * sizeof(double);
     return ((g + 255) / 256) * 256 + partials;
@@ -829,7 +885,11 @@ extern "C" AcResult acDeviceIntegrateSubstepAdjoint(const Device d, const Stream
     A.lf = lam_f;
     A.lw = lam_w;
     A.g = (AcReal*)workspace;
-    const size_t gbytes = ((size_t)A.count * NG * sizeof(AcReal) + 255) / 256 * 256;
+    const AdjLayout lay = adjoint_layout(info.int3_params[AC_nlocal]);
+    A.g_row = lay.row;
+    A.g_plane = lay.plane;
+    A.g_field = lay.field;
+    const size_t gbytes = ((size_t)lay.field * NG * sizeof(AcReal) + 255) / 256 * 256;
     A.partials = (double*)((char*)workspace + gbytes);
     hipStream_t s = device_stream(d, stream);
     launch_adjoint<AcReal>(A, info.bool_params[AC_lupwd] != 0, info.bool_params[AC_lentropy] != 0,

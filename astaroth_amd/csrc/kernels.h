@@ -67,18 +67,19 @@ bool split_shape_fits(TiledShape s, int nx, int ny, int nz);
 int split_candidates(int nx, int ny, int nz, TiledShape* out, int max_out);
 template <typename T>
 bool split_reads_periodic(const SolveArgs<T>& a, int kahan_bits, TiledShape shape);
-// The adjoint's local stage on the tiled machinery: derivative adjoints g (NG fields of m^3,
-// same field stride as the state), lambda_f / lambda_w (NF fields, updated in place at the
+// The adjoint's local stage on the tiled machinery: derivative adjoints g (NG fields, laid
+// out as AdjLayout says), lambda_f / lambda_w (NF fields, updated in place at the
 // interior cells: lambda_w <- alpha mu, lambda_f <- lambda_f + dt * the value adjoints), (nu, eta)
 // block partials.
 template <typename T>
 struct AdjLocal {
     T* g;
+    long long g_row, g_plane, g_field;  // strides of g (values)
     T* lf;
     T* lw;
     double* partials;
 };
-// Returns false (nothing launched) when the grid does not fit 64 x 4 tiles.
+// Returns false (nothing launched) when the grid does not fit 64 x 4 tiles, and in FP64.
 template <typename T>
 bool launch_adjoint_local_tiled(const SolveArgs<T>& a, const AdjLocal<T>& x, bool upwd,
                                 bool entropy, hipStream_t s, long long* nblocks);
@@ -130,21 +131,24 @@ __device__ __forceinline__ gchar* sbase(const void* p)
 {
     return (gchar*)opaque_s64((long long)p);
 }
-// z-chunk of the adjoint's local stage (64 x 4 column blocks, one 256-thread workgroup per CU):
-// long chunks amortise the six plane steps of each chunk's start-up; the longest of 256, 128
-// and 64 (up to all of nz) that still gives at least 256 workgroups, one per CU of the MI355X
-// (256^3: one 256-plane chunk per column, 9.20 -> 9.01 ms per adjoint step against 128-plane
-// chunks), else the largest of 32, 16 and 8 below nz.
+// z-chunk of the adjoint's local stage (64 x 4 column blocks, one 256-thread workgroup per CU): the
+// divisor of nz with the fewest plane steps, rounds of workgroups over the 256 CUs times the planes of a
+// chunk and the six that start it up, the longest among equals.
 inline int adjoint_zchunk(int nx, int ny, int nz)
 {
     const long long tiles = (long long)(nx / 64) * (ny / 4);
-    for (int cand : {256, 128, 64})
-        if (nz % cand == 0 && nz >= cand && tiles * (nz / cand) >= 256)
-            return cand;
-    for (int cand : {32, 16, 8})
-        if (nz % cand == 0 && nz > cand)
-            return cand;
-    return nz;
+    int best = nz;
+    long long least = 1ll << 62;
+    for (int zc = nz; zc >= 1; --zc) {
+        if (nz % zc != 0)
+            continue;
+        const long long cost = (tiles * (nz / zc) + 255) / 256 * (zc + 6);
+        if (cost < least) {
+            least = cost;
+            best = zc;
+        }
+    }
+    return best;
 }
 // Candidate launch shapes of the tiled kernels (for the autotuner).
 int tiled_num_shapes();

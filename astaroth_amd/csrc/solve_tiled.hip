@@ -219,6 +219,7 @@ __device__ __forceinline__ void delay_line_body(const SolveArgs<T>& a, const Adj
     const int gx = x0 + tx, gy = y0 + ty;
     const int ctr = (ty + R) * LX + (tx + R);
     const unsigned ioff = (unsigned)((gx + R) + (int)sy * (gy + R));  // in-plane offset
+    const unsigned goff = ADJ ? (unsigned)((gx + (int)x.g_row * gy) * (int)sizeof(T)) : 0u;  // in g, bytes
 
     dma_plane(z0 - R, 0, a.fstride * (long long)sizeof(T));
     if (LATE)
@@ -436,8 +437,11 @@ __device__ __forceinline__ void delay_line_body(const SolveArgs<T>& a, const Adj
                 pnu += (double)dt * (double)anu;
                 peta += (double)dt * (double)aeta;
                 const long long poffb = sz * (long long)(z + R) * (long long)sizeof(T);
+                const long long gfsb = opaque_s64(x.g_field * (long long)sizeof(T));
+                const long long gpb = x.g_plane * (long long)z * (long long)sizeof(T);
+                const unsigned gob = opaque(goff);
                 put_derivative_adjoints<UPWD>(ad, aup, [&](int k, T v) {
-                    st_b((T*)((char*)x.g + (k * fsb + poffb)), iob, v);
+                    st_b((T*)((char*)x.g + (k * gfsb + gpb)), gob, v);
                 });
                 // the pointwise parts of the substep's adjoint: lambda_w <- alpha mu, and
                 // lambda_f gains dt times the adjoint of the cell's own value (the transposed
@@ -823,6 +827,12 @@ template <typename T>
 bool launch_adjoint_local_tiled(const SolveArgs<T>& a, const AdjLocal<T>& x, bool upwd,
                                 bool entropy, hipStream_t s, long long* nblocks)
 {
+#if AC_DOUBLE_PRECISION
+    // FP64 takes the blocks of adjoint.hip at every size: this form holds one wave per SIMD with spills
+    // (whole adjoint substep, blocks against this: 64^3 123 against 160 us, 128^3 980 / 1000, 192^3 3265 /
+    // 3461, 256^3 7800 / 7470)
+    return false;
+#else
     if (a.nx % 64 != 0 || a.ny % 4 != 0 || !uniform_slabs(a, 0))
         return false;
     const int zc = adjoint_zchunk(a.nx, a.ny, a.nz);
@@ -834,6 +844,7 @@ bool launch_adjoint_local_tiled(const SolveArgs<T>& a, const AdjLocal<T>& x, boo
     else if (entropy) hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, false, true>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     else hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, false, false>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     return true;
+#endif
 }
 
 template bool launch_adjoint_local_tiled<AcRealT>(const SolveArgs<AcRealT>&, const AdjLocal<AcRealT>&,
