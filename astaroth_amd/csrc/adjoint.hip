@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 
+#include "block_stage.h"
 #include "kernels.h"
 #include "mhd_adjoint.h"
 
@@ -158,66 +159,24 @@ __global__ void __launch_bounds__(256) tangent_kernel(AdjArgs<T> A)
     }
 }
 
-// This wave's memory operations and LDS reads are done, then the workgroup barrier.
-__device__ __forceinline__ void memory_barrier()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // ---------------------------------------------------------------- adjoint (A): local part
 // One cell per thread on blocks of 16 x 4 x 4 cells, in FP64 and for FP32 grids that the tiled form's 64 x 4
-// columns do not divide. The block's box of the state, with its radius-3 halo, is DMA'd into LDS and all
-// stencils read it there (22 x 10 x 10 cells of 8 fields: 69 loads per cell, from L2 mostly, in place of
-// the 230 that the stencils make). 16 columns are one 64-byte line of the derivative adjoints in FP32.
+// columns do not divide. All stencils read the block's box in LDS. 16 columns are one 64-byte line of the derivative adjoints in FP32.
 // Reading the stencils from global memory it took 163 us at 72 x 60 x 50 FP64, now 70; whole adjoint
 // substep 144 x 128 x 112 FP32 1206 -> 574 us. Two workgroups share a CU in FP32 (222 VGPRs), one in FP64;
 // their load, stencil and store phases overlap only with each other's.
-constexpr int BX = 16, BY = 4, BZ = 4;
-constexpr int BLX = BX + 2 * R, BLY = BY + 2 * R, BLZ = BZ + 2 * R;
-
-static long long adjoint_local_blocks(int nx, int ny, int nz)
-{
-    return (long long)((nx + BX - 1) / BX) * ((ny + BY - 1) / BY) * ((nz + BZ - 1) / BZ);
-}
-
 template <typename T, bool UPWD, bool ENTROPY>
 __global__ void __launch_bounds__(BX * BY * BZ) adjoint_local_kernel(AdjArgs<T> A)
 {
-    constexpr int NW = BX * BY * BZ / 64;
-    constexpr int WPE = (int)sizeof(T) / 4;
-    constexpr int BOX = BLX * BLY * BLZ * WPE;                    // dwords of a field's box
-    constexpr int NR = ((BOX + 63) / 64 + NW - 1) / NW;           // DMA rounds per wave
-    constexpr int LPS = NR * NW * 64 / WPE;                       // padded field stride in LDS (values)
+    constexpr int NW = BlockStage<T>::NW, LPS = BlockStage<T>::LPS;
     __shared__ T lds[NF * LPS];
     __shared__ double sh[2][NW];
     const SolveArgs<T>& a = A.s;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // each XCD takes a contiguous range of blocks, whose neighbours then share its L2
-    const int nb = (int)gridDim.x;
-    const int bid = (nb & 7) == 0 ? ((int)blockIdx.x & 7) * (nb >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
-    const int nbx = (a.nx + BX - 1) / BX, nby = (a.ny + BY - 1) / BY;
-    const int x0 = bid % nbx * BX, y0 = bid / nbx % nby * BY, z0 = bid / (nbx * nby) * BZ;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        int d = (wave + r * NW) * 64 + lane;
-        if (d >= BOX)
-            d = 0;  // padding lanes re-read dword 0 of the box
-        const int e = d / WPE, wd = d - e * WPE;
-        const int lz = e / (BLX * BLY), ly = e / BLX % BLY, lx = e % BLX;
-        // past the array (blocks at the upper edges): the last cell, unused
-        const long long src = min(x0 + lx, a.mx - 1) + (long long)a.mx * min(y0 + ly, a.my - 1) +
-                              a.sz * min(z0 + lz, a.mz - 1);
-#pragma unroll
-        for (int q = 0; q < NF; ++q)
-            __builtin_amdgcn_global_load_lds((const void*)((const char*)(a.in[q] + src) + 4 * wd),
-                                             (lds_ptr_t)(lds + q * LPS + (wave + r * NW) * (64 / WPE)), 4, 0, 0);
-    }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int3 o0 = block_origin(a.nx, a.ny);
+    stage_block(a, o0, false, lds);
     const int tx = tid % BX, ty = tid / BX % BY, tz = tid / (BX * BY);
-    const int i = x0 + tx, j = y0 + ty, k = z0 + tz;
+    const int i = o0.x + tx, j = o0.y + ty, k = o0.z + tz;
     const bool active = i < a.nx && j < a.ny && k < a.nz;
     const long long c = active ? (long long)(i + R) + (long long)a.mx * (j + R) + a.sz * (k + R) : 0;
     T lf[NF], mu[NF];
@@ -712,7 +671,7 @@ void launch_tangent(const AdjArgs<T>& A, bool upwd, bool entropy, hipStream_t s)
 // At least the workgroups of stage (A) in either form.
 long long adjoint_num_blocks(int nx, int ny, int nz)
 {
-    return std::max((long long)((nx + 63) / 64) * ((ny + 3) / 4) * nz, adjoint_local_blocks(nx, ny, nz));
+    return std::max((long long)((nx + 63) / 64) * ((ny + 3) / 4) * nz, block_count(nx, ny, nz));
 }
 
 struct TransposeShape {
@@ -757,7 +716,7 @@ void launch_adjoint(const AdjArgs<T>& A, bool upwd, bool entropy, double* param_
     long long nb = 0;
     const AdjLocal<T> xl{A.g, A.g_row, A.g_plane, A.g_field, A.lf, A.lw, A.partials};
     if (!launch_adjoint_local_tiled<T>(A.s, xl, upwd, entropy, s, &nb)) {
-        nb = adjoint_local_blocks(A.s.nx, A.s.ny, A.s.nz);
+        nb = block_count(A.s.nx, A.s.ny, A.s.nz);
         const dim3 bpg((unsigned)nb), tpb(BX * BY * BZ);
         if (upwd && entropy) hipLaunchKernelGGL((adjoint_local_kernel<T, true, true>), bpg, tpb, 0, s, A);
         else if (upwd) hipLaunchKernelGGL((adjoint_local_kernel<T, true, false>), bpg, tpb, 0, s, A);

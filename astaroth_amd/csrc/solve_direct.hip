@@ -1,15 +1,22 @@
-// solve_direct.hip -- one cell per thread fused RK3 substep, stencil points read straight from
-// global memory (served by L1/L2). This is the simple, obviously-correct solve kernel: it is
-// the parity anchor for the LDS-tiled kernel and the fallback for grids the tiled kernel does
-// not cover. Semantics: ref acc-runtime/samples/mhd_modular/mhdsolver.ac:586-636 fused into one
-// pass (ref twopass_solve_intermediate + twopass_solve_final).
-#include "mhd_common.h"
+// solve_direct.hip -- one cell per thread fused RK3 substep. This is the simple, obviously-correct solve
+// kernel: it is the parity anchor for the marching kernels, the fallback for what they do not cover
+// (fields that are not one slab), and the kernel of FP32 gradients on grids that 64 columns do not
+// divide. STAGED: a block's stencils are read from LDS (block_stage.h); else from global memory, the
+// same arithmetic. Three substeps and fills, staged against not: 144 x 128 x 112 FP32 0.47 against 0.88 ms,
+// 100 x 75 x 50 0.147 / 0.189, 48^3 0.056 / 0.076, 40^3 0.058 / 0.058, 32^3 0.0386 / 0.0355 (latency: 128
+// blocks on 256 CUs); FP64 100 x 90 x 75 0.445 / 1.12 ms, 16^3 0.047 / 0.074, so FP64 always stages.
+// Semantics: ref acc-runtime/samples/mhd_modular/mhdsolver.ac:586-636 fused into one pass (ref
+// twopass_solve_intermediate + twopass_solve_final).
+#include <type_traits>
+
+#include "block_stage.h"
 #include "kernels.h"
+#include "mhd_common.h"
 
 namespace acamd {
 
-template <typename T>
-__device__ __forceinline__ T der1(const T* __restrict__ f, long long c, long long s, const T* k)
+template <typename T, typename I>
+__device__ __forceinline__ T der1(const T* __restrict__ f, I c, I s, const T* k)
 {
     return k[1] * (f[c + s] - f[c - s]) + k[2] * (f[c + 2 * s] - f[c - 2 * s]) +
            k[3] * (f[c + 3 * s] - f[c - 3 * s]);
@@ -17,8 +24,8 @@ __device__ __forceinline__ T der1(const T* __restrict__ f, long long c, long lon
 // Second (and upwind) derivative. CF: the cancellation-free form of the precise 32-bit mode,
 // sum_o k_o ((f_o - f_0) + (f_-o - f_0)), whose weights sum to zero like the sum form's, so the
 // centre weight drops out; differences of neighbouring values are exact in FP32.
-template <bool CF, typename T>
-__device__ __forceinline__ T der2(const T* __restrict__ f, long long c, long long s, const T* k)
+template <bool CF, typename T, typename I>
+__device__ __forceinline__ T der2(const T* __restrict__ f, I c, I s, const T* k)
 {
     if constexpr (CF) {
         const T f0 = f[c];
@@ -30,9 +37,8 @@ __device__ __forceinline__ T der2(const T* __restrict__ f, long long c, long lon
            k[3] * (f[c + 3 * s] + f[c - 3 * s]);
 }
 // Mixed derivative; CF pairs the corners as (f(o,o) - f(o,-o)) - (f(-o,o) - f(-o,-o)).
-template <bool CF, typename T>
-__device__ __forceinline__ T derm(const T* __restrict__ f, long long c, long long sa, long long sb,
-                                  const T* k)
+template <bool CF, typename T, typename I>
+__device__ __forceinline__ T derm(const T* __restrict__ f, I c, I sa, I sb, const T* k)
 {
     T r = T(0);
 #pragma unroll
@@ -47,44 +53,70 @@ __device__ __forceinline__ T derm(const T* __restrict__ f, long long c, long lon
     return r;
 }
 
-template <typename T, bool UPWD, bool ENTROPY, int KB>
-__global__ void __launch_bounds__(256) solve_direct_kernel(SolveArgs<T> a)
+// The values are computed here: the compiler otherwise reads the LDS values of many stencils ahead of
+// their sums and spills (57 registers in FP32, 162 in FP64).
+template <typename T>
+__device__ __forceinline__ void keep_here(T& a, T& b, T& c, T& d)
 {
-    const int i = threadIdx.x + blockIdx.x * blockDim.x;
-    const int j = threadIdx.y + blockIdx.y * blockDim.y;
-    const int k = blockIdx.z;
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+
+template <typename T, bool UPWD, bool ENTROPY, int KB, bool STAGED>
+__global__ void __launch_bounds__(BX * BY * BZ, (sizeof(T) == 4 && STAGED ? 2 : 1)) solve_direct_kernel(SolveArgs<T> a)
+{
+    __shared__ T lds[STAGED ? NF * BlockStage<T>::LPS : 1];
+    const int3 o = block_origin(a.nx, a.ny);
+    if constexpr (STAGED)
+        stage_block(a, o, false, lds);
+    const int tid = threadIdx.x;
+    const int tx = tid % BX, ty = tid / BX % BY, tz = tid / (BX * BY);
+    const int i = o.x + tx, j = o.y + ty, k = o.z + tz;
     const bool active = i < a.nx && j < a.ny && k < a.nz;
     // the precise mode (32-bit compensation records, FP32)
     constexpr bool CF = sizeof(T) == 4 && KB == 32;
     double u2 = 0.0;  // max |u_new|^2 (the courant timestep mode)
     const T dt = solve_dt(a);
+    if constexpr (STAGED)
+        memory_barrier();
     if (active) {
-        const long long sx = 1, sy = a.mx, sz = a.sz;
-        const long long c = (long long)(i + R) + sy * (j + R) + sz * (k + R);
-        const long long st[3] = {sx, sy, sz};
+        const long long c = (long long)(i + R) + (long long)a.mx * (j + R) + a.sz * (k + R);
+        // cell and strides where the stencils are read: in the staged box, or in the arrays
+        using I = std::conditional_t<STAGED, int, long long>;
+        const I sx = 1, sy = STAGED ? (I)BLX : (I)a.mx, sz = STAGED ? (I)(BLX * BLY) : (I)a.sz;
+        const I l = STAGED ? (I)((tx + R) + BLX * (ty + R) + BLX * BLY * (tz + R)) : (I)c;
+        const I st[3] = {sx, sy, sz};
+        const T* in[NF];
+#pragma unroll
+        for (int q = 0; q < NF; ++q)
+            in[q] = STAGED ? lds + q * BlockStage<T>::LPS : a.in[q];
         const Coeffs<T>& C = a.C;
 
         CellDerivs<T> d;
         T grad[NF][3], lap[NF], upw[4][3];
 #pragma unroll
         for (int q = 0; q < NF; ++q) {
-            const T* f = a.in[q];
+            const T* f = in[q];
 #pragma unroll
             for (int ax = 0; ax < 3; ++ax)
-                grad[q][ax] = der1(f, c, st[ax], C.d1[ax]);
-            lap[q] = der2<CF>(f, c, sx, C.d2[0]) + der2<CF>(f, c, sy, C.d2[1]) + der2<CF>(f, c, sz, C.d2[2]);
+                grad[q][ax] = der1(f, l, st[ax], C.d1[ax]);
+            lap[q] = der2<CF>(f, l, sx, C.d2[0]) + der2<CF>(f, l, sy, C.d2[1]) + der2<CF>(f, l, sz, C.d2[2]);
+            if constexpr (STAGED)
+                keep_here(grad[q][0], grad[q][1], grad[q][2], lap[q]);
         }
         if (UPWD) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 4; ++q) {
 #pragma unroll
                 for (int ax = 0; ax < 3; ++ax)
-                    upw[q][ax] = der2<CF>(a.in[q], c, st[ax], C.up[ax]);
+                    upw[q][ax] = der2<CF>(in[q], l, st[ax], C.up[ax]);
+                if constexpr (STAGED)
+                    keep_here(upw[q][0], upw[q][1], upw[q][2], lap[q]);
+            }
         }
         T val[NF];
 #pragma unroll
         for (int q = 0; q < NF; ++q)
-            val[q] = a.in[q][c];
+            val[q] = in[q][l];
 
         d.lr = val[0];
         d.laplr = lap[0];
@@ -117,16 +149,18 @@ __global__ void __launch_bounds__(256) solve_direct_kernel(SolveArgs<T> a)
         // grad div: second derivatives on the diagonal, mixed derivatives off it
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-            const T* fx = a.in[1 + 3 * v];
-            const T* fy = a.in[2 + 3 * v];
-            const T* fz = a.in[3 + 3 * v];
+            const T* fx = in[1 + 3 * v];
+            const T* fy = in[2 + 3 * v];
+            const T* fz = in[3 + 3 * v];
             T* gd = v == 0 ? d.gdu : d.gda;
-            gd[0] = der2<CF>(fx, c, sx, C.d2[0]) + derm<CF>(fy, c, sx, sy, C.mx[0]) +
-                    derm<CF>(fz, c, sx, sz, C.mx[1]);
-            gd[1] = derm<CF>(fx, c, sx, sy, C.mx[0]) + der2<CF>(fy, c, sy, C.d2[1]) +
-                    derm<CF>(fz, c, sy, sz, C.mx[2]);
-            gd[2] = derm<CF>(fx, c, sx, sz, C.mx[1]) + derm<CF>(fy, c, sy, sz, C.mx[2]) +
-                    der2<CF>(fz, c, sz, C.d2[2]);
+            gd[0] = der2<CF>(fx, l, sx, C.d2[0]) + derm<CF>(fy, l, sx, sy, C.mx[0]) +
+                    derm<CF>(fz, l, sx, sz, C.mx[1]);
+            gd[1] = derm<CF>(fx, l, sx, sy, C.mx[0]) + der2<CF>(fy, l, sy, C.d2[1]) +
+                    derm<CF>(fz, l, sy, sz, C.mx[2]);
+            gd[2] = derm<CF>(fx, l, sx, sz, C.mx[1]) + derm<CF>(fy, l, sy, sz, C.mx[2]) +
+                    der2<CF>(fz, l, sz, C.d2[2]);
+            if constexpr (STAGED)
+                keep_here(gd[0], gd[1], gd[2], lap[3 * v + 1]);
         }
 
         T rhs[NF];
@@ -149,8 +183,7 @@ __global__ void __launch_bounds__(256) solve_direct_kernel(SolveArgs<T> a)
     if (a.step == 2) {
         if (a.umax2_next != nullptr)
             wave_max_to_global(u2, a.umax2_next);
-        if (a.time_acc != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 &&
-            threadIdx.x == 0 && threadIdx.y == 0)
+        if (a.time_acc != nullptr && blockIdx.x == 0 && tid == 0)
             *a.time_acc += (double)dt;
     }
 }
@@ -158,9 +191,15 @@ __global__ void __launch_bounds__(256) solve_direct_kernel(SolveArgs<T> a)
 template <typename T, bool UPWD, bool ENTROPY, int KB>
 static void launch_direct(const SolveArgs<T>& a, hipStream_t stream)
 {
-    const dim3 tpb(64, 4, 1);
-    const dim3 bpg((a.nx + 63) / 64, (a.ny + 3) / 4, a.nz);
-    hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB>), bpg, tpb, 0, stream, a);
+    const dim3 bpg((unsigned)block_count(a.nx, a.ny, a.nz)), tpb(BX * BY * BZ);
+    if constexpr (sizeof(T) == 4) {
+        // at most one block per CU: the stencils straight from the caches
+        if (bpg.x <= 256) {
+            hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, false>), bpg, tpb, 0, stream, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, true>), bpg, tpb, 0, stream, a);
 }
 
 template <typename T>
