@@ -15,8 +15,9 @@ from checkpoints. Checkpoint schedules:
 the run with periodic halos filled, and its backward gives gradients for f0 (interior cells;
 halos receive none, since the first halo fill overwrites them), nu and eta.
 
-torch provides device memory and the synchronisation points here; every computation runs in the
-HIP kernels of astaroth_amd/lib through the C ABI.
+torch provides device memory and the ordering between its current stream and the device's stream 0
+here (events, without waiting on the host); every computation runs in the HIP kernels of
+astaroth_amd/lib through the C ABI.
 """
 import ctypes
 import functools
@@ -134,6 +135,8 @@ class MHDAdjoint:
         ws = lib.acAdjointWorkspaceBytes(self.dev.handle)
         self.workspace = torch.empty(int(ws), dtype=torch.uint8, device=self.tdev)
         self.param_grad = torch.zeros(2, dtype=torch.float64, device=self.tdev)
+        self.scratch = None  # a state's worth of memory for reverse_step
+        self.stream = torch.cuda.ExternalStream(self.dev.stream_handle(0), device=self.tdev)
         self.forward_steps = 0   # forward steps run (including recomputation), for cost reports
         self.adjoint_steps = 0
 
@@ -141,14 +144,34 @@ class MHDAdjoint:
     def _sync(self):
         ac.check(self.lib.acDeviceSynchronizeStream(self.dev.handle, ac.STREAM_ALL), "sync")
 
+    # Tensors are allocated, freed and reused in the order of torch's current stream. Every use on the
+    # device's stream lies between these two, so memory freed after it cannot be reused before it.
+    def _enter(self):
+        """Orders the device's stream after the work on torch's current stream."""
+        self.stream.wait_stream(torch.cuda.current_stream(self.tdev))
+
+    def _leave(self):
+        """Orders torch's current stream after the work on the device's stream."""
+        torch.cuda.current_stream(self.tdev).wait_stream(self.stream)
+
+    def _load(self, t):
+        self._enter()
+        ac.check(self.lib.acDeviceLoadMeshFromDevicePtr(self.dev.handle, 0, t.data_ptr()), "load")
+        self._leave()
+
+    def _store(self, t):
+        self._enter()
+        ac.check(self.lib.acDeviceStoreMeshToDevicePtr(self.dev.handle, 0, t.data_ptr()), "store")
+        self._leave()
+
     def load(self, t):
         torch.cuda.synchronize(self.tdev)
-        ac.check(self.lib.acDeviceLoadMeshFromDevicePtr(self.dev.handle, 0, t.data_ptr()), "load")
+        self._load(t)
         self._sync()
 
     def store(self, t):
         self._sync()
-        ac.check(self.lib.acDeviceStoreMeshToDevicePtr(self.dev.handle, 0, t.data_ptr()), "store")
+        self._store(t)
         self._sync()
 
     def empty(self):
@@ -167,13 +190,14 @@ class MHDAdjoint:
     def run_forward(self, f0, nu, eta):
         """Runs nsteps from f0; returns the final state (halos filled) and the checkpoints."""
         self.set_params(nu, eta)
-        self.load(f0.contiguous())
+        f0 = f0.contiguous()
+        self._load(f0)
         ckpts = {}
         if self.schedule == "uniform":
             for i in range(self.nsteps):
                 if i % self.every == 0:
                     t = self.empty()
-                    self.store(t)
+                    self._store(t)
                     ckpts[("ckpt", i)] = t
                 self.advance(1)
         else:
@@ -181,34 +205,22 @@ class MHDAdjoint:
             self.advance(self.nsteps)
         self.dev.periodic()
         out = self.empty()
-        self.store(out)
+        self._store(out)
         return out, ckpts
 
     # ---- adjoint of one step whose input state is in the device
     def reverse_step(self, lam_f, lam_w):
-        # the states entering substeps 0 and 1 are saved; the one entering substep 2 is left in
-        # the device by the recomputation, where the first adjoint substep reads it (an adjoint
-        # substep reads the device state and writes only lambda and its workspace)
-        s0 = self.empty()
-        self.store(s0)
-        states = [s0]
-        for s in range(2):
-            self.dev.periodic()
-            self.dev.substep(s, self.dt)
-            self.dev.swap()
-            if s == 0:
-                t = self.empty()
-                self.store(t)
-                states.append(t)
-        for s in (2, 1, 0):
-            if s < 2:
-                self.load(states[s])
-            self.dev.periodic()
-            ac.check(self.lib.acDeviceIntegrateSubstepAdjoint(
-                self.dev.handle, 0, s, self.dt, ctypes.c_void_p(lam_f.data_ptr()),
-                ctypes.c_void_p(lam_w.data_ptr()), ctypes.c_void_p(self.workspace.data_ptr()),
-                ctypes.c_void_p(self.param_grad.data_ptr())), "adjoint substep")
-        self._sync()
+        # the states entering substeps 1 and 2 are recomputed into the device's output fields and into
+        # scratch, where the adjoint substeps read them
+        if self.scratch is None:
+            self.scratch = self.empty()
+        self._enter()
+        ac.check(self.lib.acDeviceIntegrateStepAdjoint(
+            self.dev.handle, 0, self.dt, ctypes.c_void_p(self.scratch.data_ptr()),
+            ctypes.c_void_p(lam_f.data_ptr()), ctypes.c_void_p(lam_w.data_ptr()),
+            ctypes.c_void_p(self.workspace.data_ptr()),
+            ctypes.c_void_p(self.param_grad.data_ptr())), "adjoint step")
+        self._leave()
         self.adjoint_steps += 1
 
     def run_adjoint(self, lam_T, ckpts, nu, eta):
@@ -217,31 +229,37 @@ class MHDAdjoint:
         lam_f = fold_halo_transpose(lam_T.to(self.tdtype)).contiguous()
         lam_w = torch.zeros_like(lam_f)
         self.param_grad.zero_()
-        torch.cuda.synchronize(self.tdev)
         store = dict(ckpts)
         acts = (uniform_actions(self.nsteps, self.every) if self.schedule == "uniform"
                 else revolve_actions(self.nsteps, self.snaps))
         for act in acts:
             kind = act[0]
             if kind == "restore":
-                self.load(store[act[2]])
+                self._load(store[act[2]])
             elif kind == "advance":
                 self.advance(act[2] - act[1])
             elif kind == "store":
                 t = self.empty()
-                self.store(t)
+                self._store(t)
                 store[act[2]] = t
             elif kind == "free":
                 store.pop(act[1], None)
             elif kind == "reverse":
                 self.reverse_step(lam_f, lam_w)
-        torch.cuda.synchronize(self.tdev)
         g = zero_halos(lam_f)
         pg = self.param_grad.detach().cpu().numpy()
         return g, float(pg[0]), float(pg[1])
 
     def close(self):
         self.dev.close()
+
+    def __del__(self):
+        # the runner's own buffers may be freed under another stream than the last that used them
+        try:
+            if self.dev.handle:
+                self._sync()
+        except Exception:
+            pass
 
 
 def fold_halo_transpose(lam):

@@ -97,6 +97,7 @@ EXPORTED = [
     "acHostMeshInitFourier", "acGetRealSize", "acGetMeshInfoSize", "acGetMeshSize",
     "acGetBuildInfo",
     "acAdjointWorkspaceBytes", "acDeviceIntegrateSubstepTangent", "acDeviceIntegrateSubstepAdjoint",
+    "acDeviceIntegrateStep", "acDeviceIntegrateStepAdjoint",
     "acDeviceLoadMeshFromDevicePtr", "acDeviceStoreMeshToDevicePtr", "acDeviceInitFourier",
     "acHostAppendTimeseries", "acGetVertexBufferName", "acDeviceSetTimestepMode",
     "acDeviceWriteSnapshot", "acDeviceReadSnapshot", "acHostAppendSnapshotInfo",
@@ -273,6 +274,8 @@ class AstarothLib:
             "acDeviceUpdateTimestepCFL": [dev, i, R],
             "acDeviceGetTimestep": [dev, i, P(ctypes.c_double)],
             "acDeviceIntegrateSubstepDeviceDt": [dev, i, i, R],
+            "acDeviceIntegrateStep": [dev, i, R],
+            "acDeviceIntegrateStepAdjoint": [dev, i, R] + [ctypes.c_void_p] * 5,
             "acDeviceIntegrateStepsCFL": [dev, i, i, R, P(ctypes.c_double)],
             "acDeviceReduceDiagnostics": [dev, i, P(AcDiagnostics)],
             "acDeviceAutotune": [dev, i],
@@ -454,10 +457,7 @@ class Device:
 
     def step(self, dt, stream=STREAM_DEFAULT):
         """One full RK3 step in the reference's call pattern (samples/devicetest/main.cc:98-103)."""
-        for s in range(3):
-            self.periodic(stream)
-            self.substep(s, dt, stream)
-            self.swap()
+        check(self.lib.acDeviceIntegrateStep(self.handle, stream, dt), "acDeviceIntegrateStep")
 
     def sync(self, stream=STREAM_DEFAULT):
         check(self.lib.acDeviceSynchronizeStream(self.handle, stream), "sync")

@@ -766,6 +766,8 @@ namespace acamd {
 void device_solve_args(Device d, SolveArgs<AcRealT>& a, int step, AcRealT dt);
 hipStream_t device_stream(Device d, Stream s);
 int device_id(Device d);
+AcResult device_substep_states(Device d, hipStream_t s, AcRealT dt, AcRealT* scratch);
+void device_out_fields(Device d, const AcRealT** out);
 }  // namespace acamd
 
 using namespace acamd;
@@ -824,6 +826,32 @@ extern "C" AcResult acDeviceIntegrateSubstepTangent(const Device d, const Stream
     return hipGetLastError() == hipSuccess ? AC_SUCCESS : AC_FAILURE;
 }
 
+// The adjoint of substep `step` at the state `f` (null: the current one), halos filled.
+static AcResult adjoint_substep(const Device d, hipStream_t s, const int step, const AcReal dt, const AcReal* const* f,
+                                AcReal* lam_f, AcReal* lam_w, void* workspace, double* param_grad)
+{
+    const AcMeshInfo info = acDeviceGetLocalConfig(d);
+    const int3 m = info.int3_params[AC_mlocal];
+    AdjArgs<AcReal> A;
+    memset(&A, 0, sizeof(A));
+    device_solve_args(d, A.s, step, dt);
+    for (int q = 0; q < NF && f != nullptr; ++q)
+        A.s.in[q] = f[q];
+    A.count = (long long)m.x * m.y * m.z;
+    A.lf = lam_f;
+    A.lw = lam_w;
+    A.g = (AcReal*)workspace;
+    const AdjLayout lay = adjoint_layout(info.int3_params[AC_nlocal]);
+    A.g_row = lay.row;
+    A.g_plane = lay.plane;
+    A.g_field = lay.field;
+    const size_t gbytes = ((size_t)lay.field * NG * sizeof(AcReal) + 255) / 256 * 256;
+    A.partials = (double*)((char*)workspace + gbytes);
+    launch_adjoint<AcReal>(A, info.bool_params[AC_lupwd] != 0, info.bool_params[AC_lentropy] != 0,
+                           param_grad, s);
+    return hipGetLastError() == hipSuccess ? AC_SUCCESS : AC_FAILURE;
+}
+
 extern "C" AcResult acDeviceIntegrateSubstepAdjoint(const Device d, const Stream stream,
                                                     const int step_number, const AcReal dt,
                                                     AcReal* lam_f, AcReal* lam_w, void* workspace,
@@ -835,23 +863,27 @@ extern "C" AcResult acDeviceIntegrateSubstepAdjoint(const Device d, const Stream
     }
     if (hipSetDevice(device_id(d)) != hipSuccess)
         return AC_FAILURE;
-    const AcMeshInfo info = acDeviceGetLocalConfig(d);
-    const int3 m = info.int3_params[AC_mlocal];
-    AdjArgs<AcReal> A;
-    memset(&A, 0, sizeof(A));
-    device_solve_args(d, A.s, step_number, dt);
-    A.count = (long long)m.x * m.y * m.z;
-    A.lf = lam_f;
-    A.lw = lam_w;
-    A.g = (AcReal*)workspace;
-    const AdjLayout lay = adjoint_layout(info.int3_params[AC_nlocal]);
-    A.g_row = lay.row;
-    A.g_plane = lay.plane;
-    A.g_field = lay.field;
-    const size_t gbytes = ((size_t)lay.field * NG * sizeof(AcReal) + 255) / 256 * 256;
-    A.partials = (double*)((char*)workspace + gbytes);
+    return adjoint_substep(d, device_stream(d, stream), step_number, dt, nullptr, lam_f, lam_w, workspace, param_grad);
+}
+
+extern "C" AcResult acDeviceIntegrateStepAdjoint(const Device d, const Stream stream, const AcReal dt,
+                                                 AcReal* scratch, AcReal* lam_f, AcReal* lam_w,
+                                                 void* workspace, double* param_grad)
+{
+    if (hipSetDevice(device_id(d)) != hipSuccess)
+        return AC_FAILURE;
     hipStream_t s = device_stream(d, stream);
-    launch_adjoint<AcReal>(A, info.bool_params[AC_lupwd] != 0, info.bool_params[AC_lentropy] != 0,
-                           param_grad, s);
-    return hipGetLastError() == hipSuccess ? AC_SUCCESS : AC_FAILURE;
+    if (device_substep_states(d, s, dt, scratch) != AC_SUCCESS)
+        return AC_FAILURE;
+    const int3 m = acDeviceGetLocalConfig(d).int3_params[AC_mlocal];
+    const long long count = (long long)m.x * m.y * m.z;
+    const AcReal *second[NF], *third[NF];
+    device_out_fields(d, second);
+    for (int q = 0; q < NF; ++q)
+        third[q] = scratch + q * count;
+    const AcReal* const* f[3] = {nullptr, second, third};
+    for (int step = 2; step >= 0; --step)
+        if (adjoint_substep(d, s, step, dt, f[step], lam_f, lam_w, workspace, param_grad) != AC_SUCCESS)
+            return AC_FAILURE;
+    return AC_SUCCESS;
 }

@@ -33,6 +33,9 @@ __device__ __forceinline__ void wave_max_to_global(double v, unsigned long long*
 template <typename T>
 void launch_solve_direct(const SolveArgs<T>& a, bool upwd, bool entropy, int kahan_bits,
                          hipStream_t stream);
+// Whether it honours a.wrap on this grid (reads the periodic images instead of the halos).
+template <typename T>
+bool direct_reads_periodic(const SolveArgs<T>& a);
 
 // LDS-tiled 2.5D solve. Returns false when the launch shape does not fit the grid.
 // Tiles of 64 x 4 and 64 x 2 run the delay-line kernel (solve_tiled.hip); tiles of 32 x 8,

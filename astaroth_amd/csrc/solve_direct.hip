@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(BX * BY * BZ, (sizeof(T) == 4 && STAGED ? 2 : 
     __shared__ T lds[STAGED ? NF * BlockStage<T>::LPS : 1];
     const int3 o = block_origin(a.nx, a.ny);
     if constexpr (STAGED)
-        stage_block(a, o, false, lds);
+        stage_block(a, o, a.wrap != 0, lds);
     const int tid = threadIdx.x;
     const int tx = tid % BX, ty = tid / BX % BY, tz = tid / (BX * BY);
     const int i = o.x + tx, j = o.y + ty, k = o.z + tz;
@@ -188,13 +188,25 @@ __global__ void __launch_bounds__(BX * BY * BZ, (sizeof(T) == 4 && STAGED ? 2 : 
     }
 }
 
+// FP32 grids of at most one block per CU read the stencils straight from the caches.
+template <typename T>
+static bool staged(const SolveArgs<T>& a)
+{
+    return sizeof(T) == 8 || block_count(a.nx, a.ny, a.nz) > 256;
+}
+
+template <typename T>
+bool direct_reads_periodic(const SolveArgs<T>& a)
+{
+    return staged(a) && a.nx >= R && a.ny >= R && a.nz >= R;
+}
+
 template <typename T, bool UPWD, bool ENTROPY, int KB>
 static void launch_direct(const SolveArgs<T>& a, hipStream_t stream)
 {
     const dim3 bpg((unsigned)block_count(a.nx, a.ny, a.nz)), tpb(BX * BY * BZ);
     if constexpr (sizeof(T) == 4) {
-        // at most one block per CU: the stencils straight from the caches
-        if (bpg.x <= 256) {
+        if (!staged(a)) {
             hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, false>), bpg, tpb, 0, stream, a);
             return;
         }
@@ -220,5 +232,6 @@ void launch_solve_direct(const SolveArgs<T>& a, bool upwd, bool entropy, int kb,
 }
 
 template void launch_solve_direct<AcRealT>(const SolveArgs<AcRealT>&, bool, bool, int, hipStream_t);
+template bool direct_reads_periodic<AcRealT>(const SolveArgs<AcRealT>&);
 
 }  // namespace acamd

@@ -448,6 +448,9 @@ AcResult acDeviceGetTimestep(const Device device, const Stream stream, double* d
  * the kernel also reduces max|u| of the new state and sets the next dt (courant as given). */
 AcResult acDeviceIntegrateSubstepDeviceDt(const Device device, const Stream stream,
                                           const int step_number, const AcReal courant);
+/* One RK3 step of the given dt: periodic boundaries + fused substep + swap, three times. The result,
+ * halos included, equals that of the separate calls; `out` holds no halos. Not synchronised. */
+AcResult acDeviceIntegrateStep(const Device device, const Stream stream, const AcReal dt);
 /* nsteps full RK3 steps (periodic boundaries + fused substep + swap, three times per step) with
  * the device-resident CFL dt; no host synchronisation inside. The tiled solve kernels read the
  * periodic images of the halo cells themselves (no separate fill before their substeps; other
@@ -518,6 +521,12 @@ AcResult acDeviceIntegrateSubstepTangent(const Device device, const Stream strea
 AcResult acDeviceIntegrateSubstepAdjoint(const Device device, const Stream stream,
                                          const int step_number, const AcReal dt, AcReal* lam_f,
                                          AcReal* lam_w, void* workspace, double* param_grad);
+/* The adjoint of a whole step from the state before it (the current one, which stays): recomputes the states
+ * entering substeps 1 and 2, into `out` and into scratch (all fields, m^3 each), and runs the adjoint
+ * substeps 2, 1 and 0. w is overwritten. Not synchronised. */
+AcResult acDeviceIntegrateStepAdjoint(const Device device, const Stream stream, const AcReal dt,
+                                      AcReal* scratch, AcReal* lam_f, AcReal* lam_w, void* workspace,
+                                      double* param_grad);
 
 /* ===================== Host interface (ref include/astaroth_helpers.h, astaroth_utils.h) ===== */
 
