@@ -45,14 +45,16 @@ bool split_shape_fits(TiledShape s, int nx, int ny, int nz)
 // (six of them start a chunk up); where two workgroups share a CU, a round that has only one on each
 // takes 0.8 of the time of a full one (128 columns FP32: 1.45 against 1.8 us per plane step, measured
 // at 32^3 to 128^3). Half or twice the planes of the cheapest split cost 2-50% (128^3 FP32, 64 x 4:
-// 0.079 ms with 32 planes, 0.096 with 16, 0.14 with 64). Among splits within 3% of the cheapest
-// the shortest chunk of 32 planes or more is taken: more and shorter rounds even out when other
-// streams share the chip (256^3 FP64, launches of three streams: 1.58 ms with 128 planes, 1.66 with
-// 256; one stream: 1.41 and 1.40).
-// Blocks that cover 30% more columns than the best one are left out. So are the 128-column blocks where
-// 64 x 4 covers as few columns and has at least 16 planes to a chunk: at 128^3 FP32 32 x 4 is faster
-// alone (0.0705 against 0.079 ms), but it loses that where streams share the chip (0.088 against
-// 0.085 ms), and from 192^3 on it loses both ways.
+// 0.079 ms with 32 planes, 0.096 with 16, 0.14 with 64). Among splits within 7% of the cheapest
+// the shortest chunk of 64 planes or more is taken: more and shorter rounds keep neighbouring blocks
+// close and even out when other streams share the chip (a step, launches of three streams / of one: 512^3
+// FP32 16-bit 17.0 / 17.0 ms with 86 planes, 20.4 / 17.0 with 171, 17.7 / 17.6 with 32; 256^3 FP64 4.47 / 4.25
+// with 64, 4.75 / 4.17 with 128, 4.98 / 4.21 with 256).
+// Blocks that cover 30% more columns than the best one are left out. So are narrower blocks where a wider
+// one covers as few columns and has at least 16 planes to a chunk: at 128^3 FP32 32 x 4 is faster
+// alone than 64 x 4 (0.0705 against 0.079 ms), but it loses that where streams share the chip (0.088
+// against 0.085 ms), and from 192^3 on it loses both ways; at 256^3 FP64 16 x 8 and 32 x 4 come out even
+// alone, and 16 x 8 takes 5.1 against 4.98 ms a step with three streams.
 int split_candidates(int nx, int ny, int nz, TiledShape* out, int max_out)
 {
     long long least = 1ll << 62;
@@ -73,12 +75,12 @@ int split_candidates(int nx, int ny, int nz, TiledShape* out, int max_out)
             if (cost((nz + nch - 1) / nch) < cost(s.zchunk))
                 s.zchunk = (nz + nch - 1) / nch;
         const double least_cost = cost(s.zchunk);
-        for (int nch = 1; (nz + nch - 1) / nch >= 32; ++nch)
-            if (cost((nz + nch - 1) / nch) <= 1.03 * least_cost)
+        for (int nch = 1; (nz + nch - 1) / nch >= 64; ++nch)
+            if (cost((nz + nch - 1) / nch) <= 1.07 * least_cost)
                 s.zchunk = std::min(s.zchunk, (nz + nch - 1) / nch);
         if (split_shape_fits(s, nx, ny, nz))
             out[n++] = s;
-        if (k.tx == 64 && n > 0 && tiles * k.tx * k.ty == least && s.zchunk >= 16)
+        if (n > 0 && tiles * k.tx * k.ty == least && s.zchunk >= 16)
             break;
     }
     return n;
