@@ -1397,10 +1397,11 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
     // Candidates: the role-split shapes (any grid); in FP32 also the delay-line shapes of 64 x 4 columns
     // that give each CU its two workgroups, which are faster once the state is far larger than the caches
     // (256^3 plain: 0.54 against 0.59 ms per launch; smaller grids 0.105 against 0.079 ms at 128^3, and
-    // FP64 1.59 against 1.36 ms at 256^3), up to 2^26 cells: beyond, the trials, of single launches, come
-    // out even, and steps favour the role-split kernel (512^3 16-bit, three streams / one: 17.0 / 17.0 ms a
+    // FP64 1.59 against 1.36 ms at 256^3), except from 2^26 to 2^29 cells: the trials, of single launches, come
+    // out even there, and steps favour the role-split kernel (512^3 16-bit, three streams / one: 17.0 / 17.0 ms a
     // step against 19.0 / 17.2 for the best delay-line shape, plain 16.0 / 14.4 against 16.2 / 15.0; 384^3
-    // plain 6.6 / 6.2 against 6.7 / 6.2), except in the precise 32-bit mode (18.8 / 18.3 against 21.1 / 17.4).
+    // plain 6.6 / 6.2 against 6.7 / 6.2), if not in the precise 32-bit mode (18.8 / 18.3 against 21.1 / 17.4);
+    // at 1024^3 16-bit the delay-line kernel is ahead again (one stream 128 against 130 ms).
     // The direct kernel, at most as fast even at 16^3 to 32^3 (32^3 FP32: 0.0092 ms each) and in need of a
     // fill before each substep (22 against 33 us a step there), is tried where the configuration leaves the
     // role-split kernel out, with the delay-line and the sweep shapes of 64 columns. The ring shapes read
@@ -1414,7 +1415,8 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
         if (sh.tx != 64 || !shape_fits(sh, n))
             continue;
         const long long blocks = (long long)(n.x / 64) * (n.y / sh.ty) * (n.z / sh.zchunk);
-        const bool mid = blocks >= 512 && ((long long)n.x * n.y * n.z < (1ll << 26) || kb == 32);
+        const long long cells = (long long)n.x * n.y * n.z;
+        const bool mid = blocks >= 512 && (cells < (1ll << 26) || cells >= (1ll << 29) || kb == 32);
         if (nsplit == 0 || (sizeof(AcReal) == 4 && sh.ty == 4 && mid))
             cands.push_back(sh);
     }
