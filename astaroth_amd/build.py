@@ -17,7 +17,7 @@ OBJDIR = os.path.join(HERE, "_build")
 
 SOURCES = ["device.hip", "solve_direct.hip", "solve_tiled.hip", "solve_ring.hip", "solve_sweep.hip",
            "solve_split.hip", "solve_split_a.hip", "solve_split_b.hip", "solve_split_c.hip",
-                     "aux_kernels.hip", "ic.hip", "host.cc", "adjoint.hip", "forcing.cc", "noalloc.hip"]
+           "aux_kernels.hip", "ic.hip", "host.cc", "adjoint.hip", "forcing.cc", "noalloc.hip"]
 ARCH = os.environ.get("ASTAROTH_OFFLOAD_ARCH", "gfx950")
 
 HIP_FLAGS = [

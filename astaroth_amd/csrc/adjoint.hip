@@ -4,13 +4,13 @@
 // Tangent:  dw' = alpha_s dw + dt (J(f) df + dR/dnu dnu + dR/deta deta),  df' = df + beta_s dw'.
 // Adjoint:  mu = lw' + beta_s lf',  lw = alpha_s mu,  lf = lf' + dt J(f)^T mu,
 //           lnu += dt <mu, dR/dnu>,  leta += dt <mu, dR/deta>.
-// J^T mu is computed in three stages: (A) per cell, the adjoint of every derivative quantity
+// J^T mu is computed in two stages: (A) per cell, the adjoint of every derivative quantity
 // the right-hand side reads at a neighbour (NG = 47 fields, "derivative adjoints"), together
 // with the pointwise parts: lw = alpha mu and lf += dt * (the adjoint of the cell's own value);
-// (B) the periodic halo fill of the derivative adjoints, which is the transpose of the forward
-// halo copy; (C) per output field, the transposed stencils applied to the derivative adjoints
-// by a z-marching kernel, added to lf (first derivatives are antisymmetric, so their transpose
-// is the negative; second, upwind and mixed ones are symmetric).
+// (C) per output field, the transposed stencils applied to the derivative adjoints by a z-marching
+// kernel, added to lf (first derivatives are antisymmetric, so their transpose is the negative;
+// second, upwind and mixed ones are symmetric). Between them stands (B), the transpose of the forward
+// halo copy: (C) reads periodic images.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -615,8 +615,8 @@ __device__ __forceinline__ void transpose_block(const AdjArgs<T>& A, T* lds0, T*
 
 // All output fields in one launch: a workgroup takes one field of one column block and z-chunk. One
 // field has 64 workgroups at 128^3 (64 x 16 columns, 32 planes), a quarter of the CUs; eight launches of
-// them took 649 us FP32, this one 240, with 47 + 16 fields read or written at least once (530 MB). From
-// 256^3 on, where one field fills the chip, both are bound by the memory (1.55 ms). On grids that 64
+// them took 649 us FP32, this one 213, with 47 + 16 fields read or written at least once (530 MB). From
+// 256^3 on, where one field fills the chip, both are bound by the memory (1.4 ms). On grids that 64
 // columns do not divide, an unstaged kernel per field and a halo fill of the derivative adjoints took
 // 0.85 ms (72 x 60 x 50 FP64); this takes 60 us. The fields of one block follow each other (all blocks of
 // one field first) since neighbouring blocks in step share more than the fields of a block do (256^3
