@@ -20,7 +20,8 @@ def lib(request, require_gpu):
     return ac.load(request.param)
 
 
-@pytest.mark.parametrize("n", [(65, 17, 9), (33, 15, 7), (17, 33, 70), (31, 16, 5), (5, 4, 3), (128, 48, 67)])
+@pytest.mark.parametrize("n", [(65, 17, 9), (33, 15, 7), (17, 33, 70), (31, 16, 5), (5, 4, 3), (128, 48, 67),
+                               (160, 80, 90)])  # more blocks than the one-stage sum of the parameters takes
 @pytest.mark.parametrize("upwd,entropy,step", [(True, True, 0), (False, True, 1), (True, False, 2)])
 def test_transposes_on_any_grid(lib, n, upwd, entropy, step):
     say(f"case adjoint shapes {lib.precision} n={n} upwd={upwd} entropy={entropy} step={step}")
