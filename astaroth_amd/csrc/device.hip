@@ -251,12 +251,12 @@ static TiledShape config_shape(const AcMeshInfo& c)
                           : 0};
 }
 
-static AcResult launch_solve(Device d, const SolveArgs<AcReal>& a_in, hipStream_t s)
+// kb: the width of the compensation records that the launch reads and updates, 0 for none.
+static AcResult launch_solve(Device d, const SolveArgs<AcReal>& a_in, hipStream_t s, const int kb)
 {
     const AcMeshInfo& info = d->local_config;
     const bool upwd = info.bool_params[AC_lupwd] != 0;
     const bool entropy = info.bool_params[AC_lentropy] != 0;
-    const int kb = d->kahan_bits;
     SolveArgs<AcReal> a = a_in;
     if (a.wrap && !shape_reads_periodic(a, kb, d->shape)) {
         // the kernel that runs reads the halos: fill them first
@@ -859,7 +859,7 @@ AcResult acDeviceIntegrateSubstep(const Device d, const Stream stream, const int
         return AC_FAILURE;
     SolveArgs<AcReal> a;
     fill_solve_args(d, a, step_number, dt);
-    const AcResult r = launch_solve(d, a, s);
+    const AcResult r = launch_solve(d, a, s, d->kahan_bits);
     if (r == AC_SUCCESS && step_number == 2 && forcing_on(d))
         launch_forcing_step(d, a, s, nullptr);
     return r;
@@ -883,7 +883,7 @@ AcResult acDeviceIntegrateStep(const Device d, const Stream stream, const AcReal
         SolveArgs<AcReal> a;
         fill_solve_args(d, a, sub, dt);
         a.wrap = fill ? 0 : 1;
-        if (launch_solve(d, a, s) != AC_SUCCESS)
+        if (launch_solve(d, a, s, d->kahan_bits) != AC_SUCCESS)
             return AC_FAILURE;
         if (sub == 2 && forcing_on(d))
             launch_forcing_step(d, a, s, nullptr);
@@ -1114,7 +1114,7 @@ static AcResult substep_device_dt(Device d, hipStream_t s, const int step_number
             launch_cfl_state<AcReal>(f, d->C, n.x, n.y, n.z, d->cfl_mode, a.cfl_cs2, next, s);
         }
     }
-    const AcResult r = launch_solve(d, a, s);
+    const AcResult r = launch_solve(d, a, s, d->kahan_bits);
     if (r == AC_SUCCESS && step_number == 2 && forcing_on(d))
         launch_forcing_step(d, a, s, d->cfl_mode == 0 ? next : nullptr);
     if (step_number == 2)
@@ -1519,7 +1519,8 @@ void device_solve_args(Device d, SolveArgs<AcReal>& a, int step, AcReal dt)
     fill_solve_args(d, a, step, dt);
 }
 // The states entering the three substeps of a step, halos filled, from the current state: that one in `in`,
-// the next in `out`, the third in scratch (NF fields of m^3).
+// the next in `out`, the third in scratch (NF fields of m^3). The compensation records belong to the state
+// in `in`, so the launches are uncompensated ones, which leave them alone.
 AcResult device_substep_states(Device d, hipStream_t s, AcReal dt, AcReal* scratch)
 {
     const int3 n = d->local_config.int3_params[AC_nlocal];
@@ -1536,7 +1537,7 @@ AcResult device_substep_states(Device d, hipStream_t s, AcReal dt, AcReal* scrat
             a.in[q] = d->out[q];
             a.out[q] = third[q];
         }
-        if (launch_solve(d, a, s) != AC_SUCCESS)
+        if (launch_solve(d, a, s, 0) != AC_SUCCESS)
             return AC_FAILURE;
         launch_periodic_fill<AcReal>(sub == 0 ? d->out : third, NF, n.x, n.y, n.z, s);
     }

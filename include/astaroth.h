@@ -521,9 +521,10 @@ AcResult acDeviceIntegrateSubstepTangent(const Device device, const Stream strea
 AcResult acDeviceIntegrateSubstepAdjoint(const Device device, const Stream stream,
                                          const int step_number, const AcReal dt, AcReal* lam_f,
                                          AcReal* lam_w, void* workspace, double* param_grad);
-/* The adjoint of a whole step from the state before it (the current one, which stays): recomputes the states
- * entering substeps 1 and 2, into `out` and into scratch (all fields, m^3 each), and runs the adjoint
- * substeps 2, 1 and 0. w is overwritten. Not synchronised. */
+/* The adjoint of a whole step from the state before it (the current one, which stays, as do its compensation
+ * records): recomputes the states entering substeps 1 and 2, without compensation, into `out` and into
+ * scratch (all fields, m^3 each), and runs the adjoint substeps 2, 1 and 0. w is overwritten. Not
+ * synchronised. */
 AcResult acDeviceIntegrateStepAdjoint(const Device device, const Stream stream, const AcReal dt,
                                       AcReal* scratch, AcReal* lam_f, AcReal* lam_w, void* workspace,
                                       double* param_grad);
