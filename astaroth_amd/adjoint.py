@@ -139,6 +139,9 @@ class MHDAdjoint:
         self.stream = torch.cuda.ExternalStream(self.dev.stream_handle(0), device=self.tdev)
         self.forward_steps = 0   # forward steps run (including recomputation), for cost reports
         self.adjoint_steps = 0
+        # The workspace may hold memory that work queued on the constructor's stream still writes, and
+        # param_grad is zeroed there; the runner may be used under another stream.
+        self._enter()
 
     # ---- state movement between torch tensors and the device
     def _sync(self):
