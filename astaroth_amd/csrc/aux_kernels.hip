@@ -592,14 +592,22 @@ void launch_diagnostics(const T* const* fields, const Coeffs<T>& C, int nx, int 
 
 // ---------------------------------------------------------------- max |u|^2
 // Block-level max of a non-negative double, one atomic per workgroup at most (two per wave were most of
-// the 376 us that the reference timestep's maxima took at 128^3).
+// the 376 us that the reference timestep's maxima took at 128^3). NaNs are passed over where there are numbers.
 __device__ __forceinline__ void block_max_to_global(double v, unsigned long long* dst)
 {
     __shared__ double sh[RED_TPB / 64];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        v = fmax(v, __shfl_xor(v, off, 64));
     __syncthreads();
-    const double r = block_reduce(2, v, sh);
-    if (threadIdx.x == 0)
-        atomic_max_nonneg(dst, r);
+    if ((threadIdx.x & 63) == 0)
+        sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < RED_TPB / 64; ++w)
+            v = fmax(v, sh[w]);
+        atomic_max_nonneg(dst, v);
+    }
 }
 
 template <typename T>
@@ -752,7 +760,7 @@ __global__ void __launch_bounds__(RED_TPB) forcing_kernel(ForcingArgs<T> a, int 
     const double dt = (double)solve_dt(a.s);
     const double t0 = a.time_acc ? a.t_base + (*a.time_acc - dt) : a.t_base;
     const bool on = t0 > a.switch_time;
-    double u2 = 0.0;
+    double u2 = __builtin_nan("");  // no cell yet: an all-NaN velocity gives a NaN timestep
     // y = 2 pi xx / (ds ngrid), xx = (global index - nmin) ds
     auto part = [&](int d, int g, int ng) {
         return a.k[d] * (2.0 * M_PI * (((double)g * a.ds[d]) / (a.ds[d] * (double)ng)));

@@ -251,7 +251,9 @@ __global__ void __launch_bounds__(2 * TX* TY, (sizeof(T) == 4 ? 2 : 1))
     // in-plane offset of the column; threads outside the interior use its last row / column, so
     // their loads stay in bounds
     const unsigned ioff = (unsigned)((min(gx, a.nx - 1) + R) + sy * (min(gy, a.ny - 1) + R));
-    double u2max = 0.0;
+    // max |u_new|^2, NaN while there is no number in it: the timestep of a state whose velocity is NaN all over
+    // is NaN, as with the direct kernel
+    double u2max = __builtin_nan("");
 
     const int niter = zc + 2 * R;
     {
