@@ -1395,9 +1395,12 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
         ta[t].wrap = 1;
     }
     // Candidates: the role-split shapes (any grid); in FP32 also the delay-line shapes of 64 x 4 columns
-    // that give each CU its two workgroups, which are faster once the state is far larger than the caches
-    // (256^3 plain: 0.54 against 0.59 ms per launch; smaller grids 0.105 against 0.079 ms at 128^3, and
-    // FP64 1.59 against 1.36 ms at 256^3), except from 2^26 to 2^29 cells: the trials, of single launches, come
+    // with more than one workgroup for a CU, which holds two. They are faster once the state is far larger than the
+    // caches (256^3 plain: 0.54 against 0.59 ms per launch) and where their chunks make fewer rounds (chunks of 64
+    // planes at 192^3, 432 workgroups: 816 us a step plain against 862 for the role-split kernel and 867 for
+    // chunks of 32, precise mode 1073 against 1142 and 1155; 192 x 192 x 96 plain 426 against 474). With one
+    // workgroup per CU they lose (128^3 0.105 against 0.079 ms), as they do in FP64 (256^3 1.59 against 1.36 ms).
+    // Left out from 2^26 to 2^29 cells: the trials, of single launches, come
     // out even there, and steps favour the role-split kernel (512^3 16-bit, three streams / one: 17.0 / 17.0 ms a
     // step against 19.0 / 17.2 for the best delay-line shape, plain 16.0 / 14.4 against 16.2 / 15.0; 384^3
     // plain 6.6 / 6.2 against 6.7 / 6.2), if not in the precise 32-bit mode (18.8 / 18.3 against 21.1 / 17.4);
@@ -1406,6 +1409,7 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
     // fill before each substep (22 against 33 us a step there), is tried where the configuration leaves the
     // role-split kernel out, with the delay-line and the sweep shapes of 64 columns. The ring shapes read
     // halos as stored and never win; they stay pinnable.
+    constexpr int kCUs = 256;
     std::vector<TiledShape> cands;
     TiledShape split[4];
     const int nsplit = one_slab && !column_kernels_only(d) ? split_candidates(n.x, n.y, n.z, split, 4) : 0;
@@ -1416,8 +1420,8 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
             continue;
         const long long blocks = (long long)(n.x / 64) * (n.y / sh.ty) * (n.z / sh.zchunk);
         const long long cells = (long long)n.x * n.y * n.z;
-        const bool mid = blocks >= 512 && (cells < (1ll << 26) || cells >= (1ll << 29) || kb == 32);
-        if (nsplit == 0 || (sizeof(AcReal) == 4 && sh.ty == 4 && mid))
+        const bool tried = blocks > kCUs && (cells < (1ll << 26) || cells >= (1ll << 29) || kb == 32);
+        if (nsplit == 0 || (sizeof(AcReal) == 4 && sh.ty == 4 && tried))
             cands.push_back(sh);
     }
     if (one_slab && nsplit == 0)
