@@ -1400,11 +1400,13 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
     // planes at 192^3, 432 workgroups: 816 us a step plain against 862 for the role-split kernel and 867 for
     // chunks of 32, precise mode 1073 against 1142 and 1155; 192 x 192 x 96 plain 426 against 474). With one
     // workgroup per CU they lose (128^3 0.105 against 0.079 ms), as they do in FP64 (256^3 1.59 against 1.36 ms).
-    // Left out from 2^26 to 2^29 cells: the trials, of single launches, come
-    // out even there, and steps favour the role-split kernel (512^3 16-bit, three streams / one: 17.0 / 17.0 ms a
-    // step against 19.0 / 17.2 for the best delay-line shape, plain 16.0 / 14.4 against 16.2 / 15.0; 384^3
-    // plain 6.6 / 6.2 against 6.7 / 6.2), if not in the precise 32-bit mode (18.8 / 18.3 against 21.1 / 17.4);
-    // at 1024^3 16-bit the delay-line kernel is ahead again (one stream 128 against 130 ms).
+    // From 2^26 to 2^29 cells they are left out, if not in the precise 32-bit mode: neither kernel is ahead at all
+    // sizes there, and the trials take half a second. A step of the role-split kernel / the best delay-line shape in
+    // ms, one stream and three streams: 448^3 plain 10.0 / 10.0 and 10.8 / 10.8, 16-bit 11.9 / 11.6 and 12.9 / 12.6;
+    // 512^3 plain 14.4 / 15.0 and 16.0 / 16.2, 16-bit 17.0 / 17.2 and 17.0 / 19.0, precise 18.3 / 17.4 and 18.8 / 21.1;
+    // 640^3 plain 28.6 / 29.6 and 32.4 / 30.9, 16-bit 32.9 / 32.0 and 39.1 / 34.7; 768^3 plain 48.9 / 48.4 and
+    // 51.8 / 53.5, 16-bit 56.7 / 55.8 and 59.1 / 59.8. On both sides of it the delay-line kernel leads a little with one
+    // stream: 384^3 plain 6.3 / 6.0, 1024^3 16-bit 130 / 128.
     // The direct kernel, at most as fast even at 16^3 to 32^3 (32^3 FP32: 0.0092 ms each) and in need of a
     // fill before each substep (22 against 33 us a step there), is tried where the configuration leaves the
     // role-split kernel out, with the delay-line and the sweep shapes of 64 columns. The ring shapes read
