@@ -106,17 +106,27 @@ def timed(lib, dev, steps, warmup, courant=0.2):
 def reference_call_pattern(ac, n, steps=20, warmup=3, dt=1e-3):
     """The drop-in loop a caller of the reference API writes (ref samples/devicetest/main.cc:
     98-103): acDevicePeriodicBoundconds + acDeviceIntegrateSubstep + acDeviceSwapBuffers per
-    substep, fixed dt, FP32, no fused multi-step path. Host-timed around device syncs."""
+    substep, fixed dt, FP32, no fused multi-step path; and the same steps as one
+    acDeviceIntegrateStep call each. Host-timed around device syncs."""
     lib, dev = make_device(ac, "fp32", n)
     try:
         dt = lib.np_real(dt)
-        fixed_steps(dev, dt, warmup)
-        wall = fixed_steps(dev, dt, steps)
+
+        def separate_calls():
+            for s in range(3):
+                dev.periodic()
+                dev.substep(s, dt)
+                dev.swap()
+
+        timed_calls(dev, separate_calls, warmup)
+        wall = timed_calls(dev, separate_calls, steps)
+        whole = timed_calls(dev, lambda: dev.step(dt), steps)
     finally:
         dev.close()
     return {"cell_updates_per_s": n ** 3 * steps / wall, "steps": steps, "dt": float(dt),
             "calls": "acDevicePeriodicBoundconds + acDeviceIntegrateSubstep + "
-                     "acDeviceSwapBuffers per substep"}
+                     "acDeviceSwapBuffers per substep",
+            "acDeviceIntegrateStep_cell_updates_per_s": n ** 3 * steps / whole}
 
 
 def cpu_baseline(n=96, min_seconds=10.0, max_steps=1000):
@@ -264,11 +274,11 @@ def field_errors_gpu(ref, cand):
     return out
 
 
-def fixed_steps(dev, dt, steps):
+def timed_calls(dev, step, steps):
     dev.sync()
     t0 = time.perf_counter()
     for _ in range(steps):
-        dev.step(dt)
+        step()
     dev.sync()
     return time.perf_counter() - t0
 
