@@ -1449,17 +1449,13 @@ static AcResult autotune(Device d, hipStream_t s, bool w_dead)
     auto time_candidate = [&](TiledShape sh) -> float {
         auto launch = [&]() -> bool {
             for (int t = 0; t < ntrial; ++t) {
-                if (sh.tx <= 0) {
-                    SolveArgs<AcReal> ad = ta[t];
-                    ad.wrap = 0;  // the direct kernel reads the halos as stored
-                    launch_solve_direct<AcReal>(ad, upwd, entropy, kb, s);
-                }
-                else {
-                    SolveArgs<AcReal> at = ta[t];
-                    at.wrap = shape_reads_periodic(at, kb, sh) ? 1 : 0;
-                    if (!launch_shape(at, upwd, entropy, kb, sh, s))
-                        return false;
-                }
+                // periodic images where the kernel reads them, as stepping has it read
+                SolveArgs<AcReal> at = ta[t];
+                at.wrap = shape_reads_periodic(at, kb, sh) ? 1 : 0;
+                if (sh.tx <= 0)
+                    launch_solve_direct<AcReal>(at, upwd, entropy, kb, s);
+                else if (!launch_shape(at, upwd, entropy, kb, sh, s))
+                    return false;
             }
             return true;
         };
