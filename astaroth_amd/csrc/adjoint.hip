@@ -179,7 +179,8 @@ __global__ void __launch_bounds__(BX * BY * BZ) adjoint_local_kernel(AdjArgs<T> 
     const int i = o0.x + tx, j = o0.y + ty, k = o0.z + tz;
     const bool active = i < a.nx && j < a.ny && k < a.nz;
     const long long c = active ? (long long)(i + R) + (long long)a.mx * (j + R) + a.sz * (k + R) : 0;
-    T lf[NF], mu[NF];
+    // threads outside the grid carry zeros through the barrier: every carried register is defined
+    T lf[NF] = {}, mu[NF] = {};
     if (active) {
 #pragma unroll
         for (int q = 0; q < NF; ++q) {
