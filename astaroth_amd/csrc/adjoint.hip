@@ -160,11 +160,11 @@ __global__ void __launch_bounds__(256) tangent_kernel(AdjArgs<T> A)
 }
 
 // ---------------------------------------------------------------- adjoint (A): local part
-// One cell per thread on blocks of 16 x 4 x 4 cells, in FP64 and for FP32 grids that the tiled form's 64 x 4
-// columns do not divide. All stencils read the block's box in LDS. 16 columns are one 64-byte line of the derivative adjoints in FP32.
-// Reading the stencils from global memory it took 163 us at 72 x 60 x 50 FP64, now 70; whole adjoint
-// substep 144 x 128 x 112 FP32 1206 -> 574 us. Two workgroups share a CU in FP32 (222 VGPRs), one in FP64;
-// their load, stencil and store phases overlap only with each other's.
+// One cell per thread on blocks of 16 x 4 x 4 cells, where the tiled form does not apply: on grids that its 64 x 4
+// columns do not divide, and in FP64 where blocks are the faster form. All stencils read the block's box in LDS. 16 columns are one 64-byte line of the derivative adjoints in FP32. Reading the stencils
+// from global memory it took 163 us at 72 x 60 x 50 FP64, now 70; whole adjoint substep 144 x 128 x 112 FP32
+// 1206 -> 574 us. Two workgroups share a CU in FP32 (222 VGPRs), one in FP64; their load, stencil and store
+// phases overlap only with each other's.
 template <typename T, bool UPWD, bool ENTROPY>
 __global__ void __launch_bounds__(BX * BY * BZ) adjoint_local_kernel(AdjArgs<T> A)
 {

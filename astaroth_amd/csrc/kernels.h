@@ -82,7 +82,7 @@ struct AdjLocal {
     T* lw;
     double* partials;
 };
-// Returns false (nothing launched) when the grid does not fit 64 x 4 tiles, and in FP64.
+// Returns false (nothing launched) when the grid does not fit 64 x 4 tiles, and in FP64 where blocks are faster.
 template <typename T>
 bool launch_adjoint_local_tiled(const SolveArgs<T>& a, const AdjLocal<T>& x, bool upwd,
                                 bool entropy, hipStream_t s, long long* nblocks);

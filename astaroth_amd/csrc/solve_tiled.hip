@@ -827,24 +827,30 @@ template <typename T>
 bool launch_adjoint_local_tiled(const SolveArgs<T>& a, const AdjLocal<T>& x, bool upwd,
                                 bool entropy, hipStream_t s, long long* nblocks)
 {
-#if AC_DOUBLE_PRECISION
-    // FP64 takes the blocks of adjoint.hip at every size: this form holds one wave per SIMD with spills
-    // (whole adjoint substep, blocks against this: 64^3 123 against 160 us, 128^3 980 / 1000, 192^3 3265 /
-    // 3461, 256^3 7800 / 7470)
-    return false;
-#else
     if (a.nx % 64 != 0 || a.ny % 4 != 0 || !uniform_slabs(a, 0))
         return false;
     const int zc = adjoint_zchunk(a.nx, a.ny, a.nz);
+    const long long tiles = (long long)(a.nx / 64) * (a.ny / 4);
+#if AC_DOUBLE_PRECISION
+    // Without upwinding or without entropy this form beats the blocks of adjoint.hip (whole adjoint substep, blocks
+    // against this: no upwinding 128^3 861 / 649 us, 256^3 6834 / 4682, 320^3 13531 / 9696; no entropy 941 / 793,
+    // 7354 / 5638, 14056 / 11532), unless the start-up of short chunks eats it (64^3, chunks of 4 planes, no
+    // upwinding: 102 / 108; 128 x 64 x 64, of 8: 193 / 177). With both it spills at one wave per SIMD and wins only
+    // where its rounds of workgroups are nearly full and long, nine tenths of the plane steps being output planes
+    // (256^3 7556 / 7137, 256 x 128 x 128 1845 / 1768; 192^3 with 0.77 of them 3288 / 3376, 128^3 with 0.84
+    // 957 / 970, 320^3 with 0.89 14885 / 15259, 64^3 118 / 155).
+    const long long steps = (tiles * (a.nz / zc) + 255) / 256 * (zc + 6);
+    if (zc < 8 || (upwd && entropy && 10 * tiles * a.nz < 9 * 256 * steps))
+        return false;
+#endif
     const int ntx = a.nx / 64, nty = a.ny / 4, nch = a.nz / zc;
     const dim3 tpb(64, 4, 1), bpg((unsigned)(ntx * nty * nch), 1, 1);
-    *nblocks = (long long)ntx * nty * nch;
+    *nblocks = tiles * nch;
     if (upwd && entropy) hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, true, true>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     else if (upwd) hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, true, false>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     else if (entropy) hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, false, true>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     else hipLaunchKernelGGL((adjoint_local_tiled_kernel<T, false, false>), bpg, tpb, 0, s, a, x, zc, ntx, nty, nch);
     return true;
-#endif
 }
 
 template bool launch_adjoint_local_tiled<AcRealT>(const SolveArgs<AcRealT>&, const AdjLocal<AcRealT>&,
