@@ -390,11 +390,16 @@ struct MarchShape {
 static MarchShape march_shape(int nx, int ny, int nz)
 {
     const long long cols = ((long long)nx * ny + RED_TPB - 1) / RED_TPB;
-    // about 1024 items, of at least four planes (six more are loaded to start a chunk)
-    const long long nch = std::max(1ll, std::min(RED_MAX_BLOCKS / cols, (long long)(nz + 3) / 4));
+    // about 1024 items, of at least four planes (six more are loaded to start a chunk), or of fewer where that makes
+    // less than 96 items: a small grid waits for the march of one item, not for its memory. Up to 128 items then, since
+    // their atomics meet on one address (reference timestep's maxima FP64 with four planes / as here / up to 320 items:
+    // 16^3 9.5 / 7.1 / 7.1 us, 24 x 20 x 18 10.1 / 7.2 / 7.3, 40^3 10.6 / 9.0 / 10.3, 7 x 5 x 300 13.5 / 9.9 / 12.4)
+    long long nch = std::max(1ll, std::min(RED_MAX_BLOCKS / cols, (long long)(nz + 3) / 4));
+    if (cols * nch < 96)
+        nch = std::max(nch, std::min((long long)nz, 128 / cols));
     const int zc = (int)((nz + nch - 1) / nch);
     const long long items = cols * ((nz + zc - 1) / zc);
-    return {zc, (int)std::min<long long>(items, reduce_num_partials(nx, ny, nz))};
+    return {zc, (int)std::min<long long>(items, RED_MAX_BLOCKS)};
 }
 
 // Calls f(c, g) for every interior cell c of this workgroup, g[q][ax] = d A_q / d x_ax for q != ax.
