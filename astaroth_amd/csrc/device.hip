@@ -1554,15 +1554,17 @@ hipStream_t device_stream(Device d, Stream s) { return get_stream(d, s); }
 int device_id(Device d) { return d->id; }
 }  // namespace acamd
 
-// Copies all fields between `in` and slabs at p, in one copy where `in` is one slab (eight copies
-// of 128^3 FP32 take 53 us, one 30).
+// Copies all fields between `in` and slabs at p, in one copy where `in` is one slab of less than 512 MiB (eight
+// copies of 128^3 FP32 take 53 us, one 30; 474 MiB 203 / 190). From there on one copy is hardly faster than the eight,
+// and at most sizes slower (512 MiB 210 us with eight, 229 with one; 776 MiB 318 / 320, 1024 MiB 405 / 448, 1400 MiB
+// 551 / 636, 2115 MiB 820 / 889, 3621 MiB 1454 / 1668).
 static AcResult copy_state(Device d, hipStream_t s, char* p, bool load)
 {
     const size_t bytes = d->count * sizeof(AcReal);
     bool one_slab = true;
     for (int q = 0; q < NF; ++q)
         one_slab = one_slab && d->in[q] == d->in[0] + (size_t)q * d->count;
-    const int copies = one_slab ? 1 : NF;
+    const int copies = one_slab && bytes * NF < ((size_t)1 << 29) ? 1 : NF;
     for (int q = 0; q < copies; ++q) {
         char* f = (char*)d->in[q];
         char* o = p + q * bytes;
