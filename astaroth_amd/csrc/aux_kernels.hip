@@ -387,7 +387,7 @@ void launch_reduce(const T* const* bufs, int map, int op, int nx, int ny, int nz
 struct MarchShape {
     int zchunk, blocks;
 };
-static MarchShape march_shape(int nx, int ny, int nz)
+static MarchShape march_shape(int realsize, int nx, int ny, int nz)
 {
     const long long cols = ((long long)nx * ny + RED_TPB - 1) / RED_TPB;
     // about 1024 items, of at least four planes (six more are loaded to start a chunk), or of fewer where that makes
@@ -397,6 +397,21 @@ static MarchShape march_shape(int nx, int ny, int nz)
     long long nch = std::max(1ll, std::min(RED_MAX_BLOCKS / cols, (long long)(nz + 3) / 4));
     if (cols * nch < 96)
         nch = std::max(nch, std::min((long long)nz, 128 / cols));
+    // Chunks of 64 planes and more are split further where the last round of workgroups leaves much of the chip idle (a
+    // CU holds two in FP64, three in FP32): rounds times planes marched, six of them to start a chunk (diagnostics, one
+    // or two chunks / split: 384^3 FP64 2675 / 1779 us, 320^3 1297 / 1065, 400 x 400 x 128 929 / 685; 384^3 FP32
+    // 826 / 677). Multiples of 512 items lie evenly on the CUs (256^3 FP32, 1024 items: 207 us, split 216).
+    const long long slots = realsize == 8 ? 512 : 768;
+    const auto rounds = [&](long long c) {
+        const long long planes = (nz + c - 1) / c;
+        return (cols * ((nz + planes - 1) / planes) + slots - 1) / slots * (planes + 6);
+    };
+    long long split = nch;
+    for (long long c = nch + 1; c <= 16 && nz / c >= 16; ++c)
+        if (rounds(c) < rounds(split))
+            split = c;
+    if (nz / nch >= 64 && cols * nch % 512 != 0 && 10 * rounds(split) <= 9 * rounds(nch))
+        nch = split;
     const int zc = (int)((nz + nch - 1) / nch);
     const long long items = cols * ((nz + zc - 1) / zc);
     return {zc, (int)std::min<long long>(items, RED_MAX_BLOCKS)};
@@ -583,7 +598,7 @@ void launch_diagnostics(const T* const* fields, const Coeffs<T>& C, int nx, int 
     a.mx = nx + 2 * R;
     a.my = ny + 2 * R;
     a.partials = partials;
-    const MarchShape shape = march_shape(nx, ny, nz);
+    const MarchShape shape = march_shape((int)sizeof(T), nx, ny, nz);
     a.zchunk = shape.zchunk;
     const int nb = std::min(shape.blocks, max_partials / DIAG_SLOTS);
     if (use_index32(nx, ny, nz))
@@ -709,7 +724,7 @@ void launch_cfl_state(const T* const* fields, const Coeffs<T>& C, int nx, int ny
     a.mode = mode;
     a.cs2 = cs2;
     a.out = out;
-    const MarchShape shape = march_shape(nx, ny, nz);
+    const MarchShape shape = march_shape((int)sizeof(T), nx, ny, nz);
     a.zchunk = shape.zchunk;
     const int nb = shape.blocks;
     if (use_index32(nx, ny, nz))
