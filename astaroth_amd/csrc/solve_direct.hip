@@ -61,15 +61,27 @@ __device__ __forceinline__ void keep_here(T& a, T& b, T& c, T& d)
     asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
 
-template <typename T, bool UPWD, bool ENTROPY, int KB, bool STAGED>
+constexpr int ROW = BX * BZ;
+
+// ROWS: a workgroup takes rows of 64 cells instead of a 16 x 4 x 4 block.
+template <typename T, bool UPWD, bool ENTROPY, int KB, bool STAGED, bool ROWS>
 __global__ void __launch_bounds__(BX * BY * BZ, (sizeof(T) == 4 && STAGED ? 2 : 1)) solve_direct_kernel(SolveArgs<T> a)
 {
     __shared__ T lds[STAGED ? NF * BlockStage<T>::LPS : 1];
-    const int3 o = block_origin(a.nx, a.ny);
-    if constexpr (STAGED)
-        stage_block(a, o, a.wrap != 0, lds);
+    constexpr int UX = ROWS ? ROW : BX, UY = BY, UZ = ROWS ? 1 : BZ;
+    static_assert(!(STAGED && ROWS) && UX * UY * UZ == BX * BY * BZ, "one thread per cell");
+    int3 o;
+    if constexpr (!ROWS) {
+        o = block_origin(a.nx, a.ny);
+        if constexpr (STAGED)
+            stage_block(a, o, a.wrap != 0, lds);
+    }
+    else {
+        const int nbx = (a.nx + UX - 1) / UX, nby = (a.ny + UY - 1) / UY, b = (int)blockIdx.x;
+        o = make_int3(b % nbx * UX, b / nbx % nby * UY, b / (nbx * nby));
+    }
     const int tid = threadIdx.x;
-    const int tx = tid % BX, ty = tid / BX % BY, tz = tid / (BX * BY);
+    const int tx = tid % UX, ty = tid / UX % UY, tz = tid / (UX * UY);
     const int i = o.x + tx, j = o.y + ty, k = o.z + tz;
     const bool active = i < a.nx && j < a.ny && k < a.nz;
     // the precise mode (32-bit compensation records, FP32)
@@ -207,11 +219,17 @@ static void launch_direct(const SolveArgs<T>& a, hipStream_t stream)
     const dim3 bpg((unsigned)block_count(a.nx, a.ny, a.nz)), tpb(BX * BY * BZ);
     if constexpr (sizeof(T) == 4) {
         if (!staged(a)) {
-            hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, false>), bpg, tpb, 0, stream, a);
+            // Rows, whose loads are wider, unless they make twice the workgroups (a step, rows / blocks: 300 x 5 x 7 37.0 /
+            // 41.4 us, 33 x 33 x 20 35.6 / 40.9, 24 x 20 x 18 34.0 / 36.0; 32^3 35.0 / 34.6, 8^3 45 / 33, 7 x 5 x 300 90 / 47)
+            const long long rows = (long long)((a.nx + ROW - 1) / ROW) * ((a.ny + BY - 1) / BY) * a.nz;
+            if (rows < 2 * block_count(a.nx, a.ny, a.nz))
+                hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, false, true>), dim3((unsigned)rows), tpb, 0, stream, a);
+            else
+                hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, false, false>), bpg, tpb, 0, stream, a);
             return;
         }
     }
-    hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, true>), bpg, tpb, 0, stream, a);
+    hipLaunchKernelGGL((solve_direct_kernel<T, UPWD, ENTROPY, KB, true, false>), bpg, tpb, 0, stream, a);
 }
 
 template <typename T>
