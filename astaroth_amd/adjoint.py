@@ -16,8 +16,8 @@ the run with periodic halos filled, and its backward gives gradients for f0 (int
 halos receive none, since the first halo fill overwrites them), nu and eta.
 
 torch provides device memory and the ordering between its current stream and the device's stream 0
-here (events, without waiting on the host); every computation runs in the HIP kernels of
-astaroth_amd/lib through the C ABI.
+here (events, without waiting on the host), and folds and clears the halos of lambda; every other
+computation runs in the HIP kernels of astaroth_amd/lib through the C ABI.
 """
 import ctypes
 import functools

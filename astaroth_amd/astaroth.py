@@ -456,7 +456,8 @@ class Device:
         check(self.lib.acDeviceSwapBuffers(self.handle), "acDeviceSwapBuffers")
 
     def step(self, dt, stream=STREAM_DEFAULT):
-        """One full RK3 step in the reference's call pattern (samples/devicetest/main.cc:98-103)."""
+        """One full RK3 step as one call (acDeviceIntegrateStep): the state and halos that the reference's
+        loop of fill, substep and swap (samples/devicetest/main.cc:98-103) leaves, with two fills less."""
         check(self.lib.acDeviceIntegrateStep(self.handle, stream, dt), "acDeviceIntegrateStep")
 
     def sync(self, stream=STREAM_DEFAULT):

@@ -3,20 +3,24 @@
 //
 // Same semantics as solve_direct.hip (ref acc-runtime/samples/mhd_modular/mhdsolver.ac:586-636 in
 // one fused pass), on any grid. A workgroup owns a TX x TY column block and marches a z-chunk, with
-// one xy plane of all eight fields (radius-3 halo) in LDS per step, double-buffered by
-// global -> LDS DMA. Its threads come in two roles of TX * TY each, one column per thread and role:
+// one xy plane of all eight fields (radius-3 halo) in LDS per step, brought there by global -> LDS
+// DMA into three plane buffers in rotation. Its threads come in two roles of TX * TY each, one column per thread and role:
 //   hydro     lnrho, u: derivatives, right-hand sides (less the magnetic thread's force) and updates;
 //   magnetic  A, ss: derivatives, right-hand sides and updates; the Lorentz force, the entropy part
 //             of the pressure force and the exponentials of the cell.
 // The two threads of a column hand each other the dozen values the other needs through LDS.
 // Holding one half of a column's carried state each (about 90 values instead of 170), the threads
 // fit a register budget at which twice as many waves are resident, which is what the z-march needs:
-// it is bound by VALU issue, and with two waves per SIMD the VALU idles whenever both wait.
+// in FP32 it is bound by VALU issue, and with two waves per SIMD the VALU idles whenever both wait. In FP64, at one
+// wave per SIMD, it is bound by that wave's waits: 256^3 issues vector instructions in 27-36% of its cycles.
 //
 // One barrier per plane step. Before it, with plane p = z + 3 just landed: chain pushes, in-plane
 // derivatives of plane p, and all of output plane z that needs no exchange value (those are
-// double-buffered by step parity, so a wave one step ahead writes the other slot). After it: the DMA
-// of plane p + 2 into the buffer just released, and the updates and stores of plane z.
+// double-buffered by step parity, so a wave one step ahead writes the other slot). After it: the
+// updates and stores of plane z, the loads of the next output's w and compensation, and last the DMA of
+// plane p + 3 into the buffer just released. The wait before a barrier counts on that order: it leaves only the
+// newest operations in flight, which are the DMA of plane p + 2 issued at the end of the step before, so plane
+// p + 1 has landed.
 #pragma once
 
 #include "kernels.h"

@@ -467,7 +467,7 @@ AcResult acDeviceReduceDiagnostics(const Device device, const Stream stream, AcD
 AcResult acDeviceAutotune(const Device device, const Stream stream);
 /* Reports the solve-kernel launch shape in use (tile_x, tile_y, zchunk). */
 AcResult acDeviceGetSolveLaunchShape(const Device device, int* tile_x, int* tile_y, int* zchunk);
-/* Reports which solve kernel that shape runs: -1 direct, 0 delay-line, 1 unrolled sweep. */
+/* Reports which solve kernel that shape runs: -1 direct, 0 delay-line or ring, 1 unrolled sweep, 2 role-split. */
 AcResult acDeviceGetSolveKernel(const Device device, int* kind);
 /* Raw device pointers of one field: in (current state), out (next state), w (RK register). */
 AcResult acDeviceGetVertexBufferPtrs(const Device device, const VertexBufferHandle vtxbuf,
